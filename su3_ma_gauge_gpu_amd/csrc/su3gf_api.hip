@@ -405,8 +405,8 @@ gf_status gf_project(const gf_lattice *lat, void *U, void *stream)
     int64_t V;
     GF_TRY(check_lattice(lat, &V));
     if (!U) return fail(GF_ERR_BAD_ARG, "U is null");
-    hipError_t e = lat->dtype == GF_F64 ? exact::launch_project<double>(lat->layout, 4, (double *)U, V, S(stream))
-                                        : exact::launch_project<float>(lat->layout, 4, (float *)U, V, S(stream));
+    hipError_t e = lat->dtype == GF_F64 ? exact::launch_project<double>(lat->layout, (double *)U, V, S(stream))
+                                        : exact::launch_project<float>(lat->layout, (float *)U, V, S(stream));
     if (e != hipSuccess) return hip_fail(e, "project kernel launch");
     return GF_OK;
 }
@@ -1535,7 +1535,7 @@ gf_status fused_phase(const gf_lattice *lat, R *U, float *gacc, int gauge, float
         a.sweep = it;
         a.parity = parity;
         a.partial = partial;
-        return fast::launch_sweep<R>(lat->layout, gauge, GF_OR, theta, gacc != nullptr, a, s);
+        return fast::launch_sweep<R>(lat->layout, gauge, theta, gacc != nullptr, a, s);
     };
     auto two_kernels = [](int) { return hipErrorNotSupported; };
     return fused_loop(lat->dims, V, gauge, tol, maxiter, check_every, coarse_every, stall_limit, exact_end, near,
@@ -1549,8 +1549,8 @@ gf_status project_unless_done(const gf_lattice *lat, void *U, const DevState *st
 {
     int64_t V = 1;
     for (int i = 0; i < 4; i++) V *= lat->dims[i];
-    hipError_t e = lat->dtype == GF_F64 ? exact::launch_project<double>(lat->layout, 4, (double *)U, V, s, st)
-                                        : exact::launch_project<float>(lat->layout, 4, (float *)U, V, s, st);
+    hipError_t e = lat->dtype == GF_F64 ? exact::launch_project<double>(lat->layout, (double *)U, V, s, st)
+                                        : exact::launch_project<float>(lat->layout, (float *)U, V, s, st);
     if (e != hipSuccess) return hip_fail(e, "project kernel launch");
     return GF_OK;
 }
@@ -1594,7 +1594,7 @@ gf_status final_quality_t(const gf_lattice *lat, R *U, int gauge, FusedCtx &fc, 
     for (int par = 0; par < 2; par++) {
         a.parity = par;
         a.partial = par ? fc.odd() : fc.even();
-        HIP_TRY(fast::launch_sweep<R>(lat->layout, gauge, GF_OR, 3, false, a, s));
+        HIP_TRY(fast::launch_sweep<R>(lat->layout, gauge, 3, false, a, s));
     }
     HIP_TRY(launch_fused_check(fc.st, fc.even(), fc.odd(), nb, check_segments(lat->dims, gauge), 0, CHECK_PRE, s));
     GF_TRY(fc.read(s));
@@ -1774,12 +1774,12 @@ gf_status gf_time_sweeps(const gf_lattice *lat, void *U, int gauge, int nsweeps,
                     SweepArgs<double> a{};
                     a.U = tiles.p; a.Udw = a.U; a.state = fc.st; a.g = geo; a.param = 1.7f; a.nsb = 32;
                     a.sweep = first + it; a.parity = par; a.partial = partial;
-                    HIP_TRY(fast::launch_sweep<double>(kTiled12, gauge, GF_OR, par + 1, false, a, s));
+                    HIP_TRY(fast::launch_sweep<double>(kTiled12, gauge, par + 1, false, a, s));
                 } else if (variant <= 1) {
                     SweepArgs<float> a{};
                     a.U = (float *)U; a.Udw = a.U; a.gacc = gb.p; a.state = fc.st; a.g = geo; a.param = 1.7f;
                     a.nsb = 32; a.sweep = first + it; a.parity = par; a.partial = partial;
-                    HIP_TRY(fast::launch_sweep<float>(12, gauge, GF_OR, variant == 0 ? par + 1 : 0, variant == 1, a,
+                    HIP_TRY(fast::launch_sweep<float>(12, gauge, variant == 0 ? par + 1 : 0, variant == 1, a,
                                                       s));
                 } else {
                     GaugeSweepArgs a{};
@@ -1882,7 +1882,7 @@ gf_status gf_run_mixed(const gf_lattice *lat, void *U, int gauge, float omega, f
                 HIP_TRY(launch_project_gauge(g, V, s));
                 HIP_TRY(launch_gauge_apply((const double *)U, lat->layout, g, b.U32, GF_F32, 12, geo, s));
             } else if (reproject > 0 && it % reproject == 0) {
-                HIP_TRY(exact::launch_project<float>(12, 4, (float *)b.U32, V, s));
+                HIP_TRY(exact::launch_project<float>(12, (float *)b.U32, V, s));
             }
             return GF_OK;
         };

@@ -164,37 +164,85 @@ __device__ __forceinline__ LinkRef<float> gauge_ref(float *g, int64_t i)
     return l;
 }
 
-template <typename R> __device__ __forceinline__ void load12(const LinkRef<R> &l, M3<R> &u)
+// NT: past the caches (a link streamed by kept_link below)
+template <bool NT, typename R> __device__ __forceinline__ R read_real(const R *p)
+{
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+template <bool NT, typename R> __device__ __forceinline__ void write_real(R *p, R v)
+{
+    if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+
+template <bool NT = false, typename R> __device__ __forceinline__ void load12(const LinkRef<R> &l, M3<R> &u)
 {
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int j = 0; j < 3; j++) {
             const int comp = 2 * (j + 3 * i);
-            u.e[i][j] = cx(l.p[l.V * comp], l.p[l.V * (comp + 1)]);
+            u.e[i][j] = cx(read_real<NT>(&l.p[l.V * comp]), read_real<NT>(&l.p[l.V * (comp + 1)]));
         }
 }
 
-template <typename R> __device__ __forceinline__ void store12(const LinkRef<R> &l, const M3<R> &u)
+template <bool NT = false, typename R> __device__ __forceinline__ void store12(const LinkRef<R> &l, const M3<R> &u)
 {
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int j = 0; j < 3; j++) {
             const int comp = 2 * (j + 3 * i);
-            l.p[l.V * comp] = u.e[i][j].x;
-            l.p[l.V * (comp + 1)] = u.e[i][j].y;
+            write_real<NT>(&l.p[l.V * comp], u.e[i][j].x);
+            write_real<NT>(&l.p[l.V * (comp + 1)], u.e[i][j].y);
         }
 }
 
-template <typename R> __device__ __forceinline__ void store_row2(const LinkRef<R> &l, const M3<R> &u)
+template <bool NT = false, typename R> __device__ __forceinline__ void store_row2(const LinkRef<R> &l, const M3<R> &u)
 {
 #pragma unroll
     for (int j = 0; j < 3; j++) {
         const int comp = 2 * (j + 6);
-        l.p[l.V * comp] = u.e[2][j].x;
-        l.p[l.V * (comp + 1)] = u.e[2][j].y;
+        write_real<NT>(&l.p[l.V * comp], u.e[2][j].x);
+        write_real<NT>(&l.p[l.V * (comp + 1)], u.e[2][j].y);
     }
+}
+
+// A link kept in the caches or streamed past them, `kept` uniform over the
+// wave.  The asm holds no instruction: without it the compiler merges the two
+// branches' loads (or stores) into one that has lost the policy.
+template <typename F, typename G> __device__ __forceinline__ void by_policy(bool kept, F cached, G streamed)
+{
+    if (kept) {
+        cached();
+    } else {
+        asm volatile("; streamed" ::: "memory");
+        streamed();
+        asm volatile("; streamed" ::: "memory");
+    }
+}
+template <typename R> __device__ __forceinline__ void load12(const LinkRef<R> &l, M3<R> &u, bool kept)
+{
+    by_policy(kept, [&] { load12<false>(l, u); }, [&] { load12<true>(l, u); });
+}
+template <typename R> __device__ __forceinline__ void store12(const LinkRef<R> &l, const M3<R> &u, bool kept)
+{
+    by_policy(kept, [&] { store12<false>(l, u); }, [&] { store12<true>(l, u); });
+}
+
+// Links beyond the Infinity Cache.  Swept in order, half-sweep after
+// half-sweep, a configuration larger than the cache evicts each link before
+// it is used again and gets nothing from it.  So the first `keep` links of
+// each parity (direction by direction) are accessed as usual and stay
+// resident, and the others are streamed past the caches (kept_links on the
+// host).  i: the site's index within its parity; both ends of a link give
+// the same answer, up to the one tile of 64 sites that a wave may straddle:
+// its first active lane decides for the wave.
+__device__ __forceinline__ bool kept_link(int64_t keep, int64_t Vh, int64_t i, int mu)
+{
+    const int64_t k = Vh * mu + i;
+    return (int64_t)__builtin_amdgcn_readfirstlane((int)(k >> 6)) < (keep >> 6);
 }
 
 // ----------------------------------------------------------- geometry

@@ -59,7 +59,22 @@ template <typename R> struct SweepArgs {
     float param;   // OR/SR parameter or SA temperature
     uint32_t seed, counter;
     int64_t nsb;   // sites per block of the reference launch (RNG key)
+    int64_t keep;  // set by the launcher: the links of each parity kept in the Infinity Cache (kept_link)
 };
+
+// The links of each parity that a sweep keeps in the 256 MB Infinity Cache
+// (kept_link), `bytes` those that a sweep touches and uses again: all of
+// 4 Vh where they fit, 208 MB of them otherwise.  FP64 OR half-sweeps, keeping
+// 256 / 208 / 150 / 0 MB, against every link cached: 32^4 144 / 136 / 135 /
+// 154 us against 162, 36^4 225 / 226 / 228 / 290 against 290, 48^4 770 / 760
+// / 779 / 828 against 955; FP32 48^4 416 / 414 / 435 / 491 against 474.
+// 28^4 (236 MB) is fastest with every link cached (86 us; 90 keeping 200 MB).
+constexpr int64_t kInfinityCacheBytes = int64_t(256) << 20, kKeptBytes = int64_t(208) << 20;
+inline int64_t kept_links(int64_t Vh, int64_t bytes)
+{
+    if (bytes <= kInfinityCacheBytes) return 4 * Vh;
+    return (int64_t)((double)(4 * Vh) * (double)kKeptBytes / (double)bytes);
+}
 
 template <typename R> struct QualityArgs {
     const R *U;
@@ -200,7 +215,7 @@ template <typename R> hipError_t launch_sweep(int stride, int gauge, int algo, c
 // st: if given, the kernel does nothing once st->done is set (a driver's
 // reprojection enqueued after the sweep that converged)
 template <typename R>
-hipError_t launch_project(int stride, int nfields, R *U, int64_t V, hipStream_t s, const DevState *st = nullptr);
+hipError_t launch_project(int stride, R *U, int64_t V, hipStream_t s, const DevState *st = nullptr);
 template <typename R> hipError_t launch_set_hot(R *U, int64_t V, uint32_t seed, uint32_t counter, hipStream_t s);
 template <typename R> hipError_t launch_quality(int stride, int gauge, const QualityArgs<R> &a, hipStream_t s);
 int64_t quality_blocks(int64_t V);
@@ -208,10 +223,11 @@ int64_t quality_blocks(int64_t V);
 
 // fast translation unit (contracted, fused theta, gauge accumulation)
 namespace fast {
-// theta: 0 none, 1 pre-update (even kernel), 2 post-update (odd kernel),
-// 3 read-only theta pass (OR only; runs only while state->near is set)
+// overrelaxation, the drivers' link sweep.  theta: 0 none, 1 pre-update (even
+// kernel), 2 post-update (odd kernel), 3 read-only theta pass (runs only
+// while state->near is set)
 template <typename R>
-hipError_t launch_sweep(int stride, int gauge, int algo, int theta, bool gacc, const SweepArgs<R> &a, hipStream_t s);
+hipError_t launch_sweep(int stride, int gauge, int theta, bool gacc, const SweepArgs<R> &a, hipStream_t s);
 }  // namespace fast
 
 // utility kernels (su3gf_kernels.hip)
