@@ -671,12 +671,16 @@ std::array<int, 8> slab_key(const Geom &geo, int gauge, int links, bool fp64)
     return {geo.N[0], geo.N[1], geo.N[2], geo.N[3], gauge, links, fp64 ? 1 : 0, geo.slice_bps ? 1 : 0};
 }
 
-// timeslices each XCD walks in the launcher's timeslice order (launch_gsweep's
-// remap = 2), or 0 where that order does not apply
-int xcd_slices(const Geom &geo)
+// the block orders (order_span) that the tuner tries beside the default: the
+// other passes of an XCD's own timeslices, or, where Nt / 8 is not whole, the
+// other divisors of Nt up to 18
+std::vector<int> order_candidates(int Nt)
 {
-    const int64_t half_slice = geo.Vh / geo.N[0];
-    return geo.N[0] % 8 == 0 && half_slice % 64 == 0 ? geo.N[0] / 8 : 0;
+    std::vector<int> out;
+    const int def = order_span(Nt, 0), top = Nt % 8 == 0 ? Nt / 8 : std::min(Nt, 18);
+    for (int P = 1; P <= top; P++)
+        if (P != def && order_span(Nt, P) == P) out.push_back(P);
+    return out;
 }
 
 // average ms of one sweep over `n` sweeps (after one unmeasured), slab 0 = two kernels
@@ -752,13 +756,11 @@ GsweepTuning tune_gsweep(const GaugeSweepArgs &ga, int gauge, bool fp64, hipStre
         const float base = time_gsweep(t, gauge, fp64, 0, n, s, ev.a, ev.b);
         if (log) std::fprintf(stderr, "su3gf tune:   two kernels, one pass: %.4f ms per sweep (%d sweeps)\n", base, n);
         float two = base;
-        const int spx = xcd_slices(geo);
-        if (g_tpass_setting < 0 && spx > 1 && base > 0) {
-            for (int P = 1; P < spx; P++) {
-                if (spx % P != 0) continue;
+        if (g_tpass_setting < 0 && base > 0) {
+            for (int P : order_candidates(geo.N[0])) {
                 t.tpass = P;
                 const float ms = time_gsweep(t, gauge, fp64, 0, n, s, ev.a, ev.b);
-                if (log) std::fprintf(stderr, "su3gf tune:   two kernels, passes of %d timeslices: %.4f\n", P, ms);
+                if (log) std::fprintf(stderr, "su3gf tune:   two kernels, %d timeslices together: %.4f\n", P, ms);
                 if (ms > 0 && ms < two && ms < 0.97f * base) {
                     two = ms;
                     tu.tpass = P;
@@ -865,14 +867,10 @@ int quality_tpass(const gf_lattice *lat, int gauge, const void *U, hipStream_t s
                                  gauge};
     const auto hit = g_quality_cache.find(key);
     if (hit != g_quality_cache.end()) return hit->second;
-    int64_t V = 1;
-    for (int d = 0; d < 4; d++) V *= lat->dims[d];
-    const int64_t half_slice = V / 2 / lat->dims[0];
-    const int spx = lat->dims[0] % 8 == 0 && half_slice % 128 == 0 && exact::quality_blocks(V) % 8 == 0
-                        ? lat->dims[0] / 8 : 0;
+    const std::vector<int> spans = order_candidates(lat->dims[0]);
     int best = 0;
     EventPair ev;
-    if (spx > 1 && hipEventCreate(&ev.a) == hipSuccess && hipEventCreate(&ev.b) == hipSuccess) {
+    if (!spans.empty() && hipEventCreate(&ev.a) == hipSuccess && hipEventCreate(&ev.b) == hipSuccess) {
         auto time = [&](int P) -> float {
             if (quality_kernel(lat, gauge, U, nullptr, nullptr, nullptr, 0, P, s) != hipSuccess) return -1.f;
             if (hipEventRecord(ev.a, s) != hipSuccess) return -1.f;
@@ -886,8 +884,8 @@ int quality_tpass(const gf_lattice *lat, int gauge, const void *U, hipStream_t s
         };
         const float one_pass = time(0);
         float best_ms = one_pass;
-        for (int P = 1; P < spx && one_pass > 0; P++) {
-            if (spx % P != 0) continue;
+        for (int P : spans) {
+            if (one_pass <= 0) break;
             const float ms = time(P);
             if (ms > 0 && ms < best_ms && ms < 0.97f * one_pass) {
                 best_ms = ms;
@@ -1099,7 +1097,6 @@ extern "C" gf_status gf_run_sa(const gf_lattice *lat, void *U, void *Udw, int ga
         ga.U0 = bU32.as<const float>();
         ga.g = bg.as<float>();
         ga.geo = geo;
-        ga.remap = 1;
         ga.seed = (uint32_t)seed;
         ga.nsb = 32;
         // (a captured schedule keeps the two-kernel sweeps: the pipelined
@@ -1734,7 +1731,7 @@ gf_status gf_time_sweeps(const gf_lattice *lat, void *U, int gauge, int nsweeps,
     GaugeSweepArgs wa{};  // variant 6: whole sweeps as the mixed run's FP32 phase runs them
     PipeBuf pipe;
     if (variant == 6) {
-        wa.U0 = pbuf.as<const float>(); wa.g = gb.p; wa.geo = geo; wa.param = 1.7f; wa.remap = 1; wa.links24 = 1;
+        wa.U0 = pbuf.as<const float>(); wa.g = gb.p; wa.geo = geo; wa.param = 1.7f; wa.links24 = 1;
         HIP_TRY(pipe.init(geo, gauge, false, s));
         wa.pipe = pipe.get();
         wa.pipe_count = &pipe.count;
@@ -1744,7 +1741,7 @@ gf_status gf_time_sweeps(const gf_lattice *lat, void *U, int gauge, int nsweeps,
     if ((variant >= 2 && variant <= 4) || variant == 7) {
         GaugeSweepArgs t{};
         t.U0 = variant == 7 ? (const float *)tiles.p : variant == 4 ? pbuf.as<const float>() : (const float *)U;
-        t.g = gb.p; t.geo = geo; t.param = 1.7f; t.remap = 1; t.links24 = variant == 4; t.links64 = variant == 7;
+        t.g = gb.p; t.geo = geo; t.param = 1.7f; t.links24 = variant == 4; t.links64 = variant == 7;
         (void)wavefront_slab(t, gauge, variant == 3 || variant == 7, s);
         tpass = t.tpass;
     }
@@ -1768,7 +1765,7 @@ gf_status gf_time_sweeps(const gf_lattice *lat, void *U, int gauge, int nsweeps,
                 if (variant == 7) {
                     GaugeSweepArgs a{};
                     a.U0 = (const float *)tiles.p; a.g = gb.p; a.links64 = 1; a.state = fc.st; a.partial = partial;
-                    a.geo = geo; a.parity = par; a.param = 1.7f; a.remap = 1; a.tpass = tpass;
+                    a.geo = geo; a.parity = par; a.param = 1.7f; a.tpass = tpass;
                     HIP_TRY(launch_gsweep(gauge, GF_OR, par + 1, true, a, s));
                 } else if (lat->dtype == GF_F64) {
                     SweepArgs<double> a{};
@@ -1786,7 +1783,7 @@ gf_status gf_time_sweeps(const gf_lattice *lat, void *U, int gauge, int nsweeps,
                     const bool q24 = variant == 4;
                     a.U0 = q24 ? pbuf.as<const float>() : (const float *)U;
                     a.g = gb.p; a.state = fc.st; a.partial = partial; a.geo = geo;
-                    a.parity = par; a.param = 1.7f; a.remap = 1; a.links24 = q24; a.tpass = tpass;
+                    a.parity = par; a.param = 1.7f; a.links24 = q24; a.tpass = tpass;
                     HIP_TRY(launch_gsweep(gauge, GF_OR, 0, variant == 3, a, s));
                 }
             }
@@ -1897,7 +1894,6 @@ gf_status gf_run_mixed(const gf_lattice *lat, void *U, int gauge, float omega, f
         ga.state = fc.st;
         ga.geo = geo;
         ga.param = omega;
-        ga.remap = 1;
         ga.links24 = mode == GF_MIXED_GAUGE24;
         PipeBuf pipe;
         HIP_TRY(pipe.init(geo, gauge, false, s));
@@ -1988,7 +1984,6 @@ gf_status gf_run_mixed(const gf_lattice *lat, void *U, int gauge, float omega, f
         gd.state = fc.st;
         gd.geo = geo;
         gd.param = omega;
-        gd.remap = 1;
         gd.links64 = 1;
         auto launch64 = [&](int parity, int theta, double *partial, int) {
             gd.parity = parity;

@@ -15,6 +15,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "su3gf_order.h"
+
 namespace su3gf {
 
 // ----------------------------------------------------------------- complex
@@ -246,28 +248,6 @@ __device__ __forceinline__ bool kept_link(int64_t keep, int64_t Vh, int64_t i, i
 }
 
 // ----------------------------------------------------------- geometry
-// Division by a runtime constant d < 2^31 for dividends n < 2^31:
-// q = (umulhi(n, m) + n) >> s with s = ceil(log2 d), m = 2^32 (2^s - d)/d + 1.
-struct FastDiv {
-    uint32_t d, m, s;
-};
-
-__device__ __forceinline__ uint32_t fdiv(uint32_t n, const FastDiv &f)
-{
-    return (__umulhi(n, f.m) + n) >> f.s;
-}
-
-// the multiplier and shift of fdiv for divisor d (1 <= d < 2^31)
-inline FastDiv make_fastdiv(uint32_t d)
-{
-    FastDiv f;
-    f.d = d;
-    f.s = 0;
-    while ((1ull << f.s) < d) f.s++;
-    f.m = (uint32_t)(((1ull << 32) * ((1ull << f.s) - d)) / d + 1);
-    return f;
-}
-
 struct Geom {
     int N[4];          // {Nt, Nx, Ny, Nz}
     int64_t V, Vh;

@@ -169,9 +169,9 @@ template hipError_t launch_set_hot<double>(double *, int64_t, uint32_t, uint32_t
 // sites of parity-split index [128 L, 128 L + 128), i.e. 256 consecutive
 // sites of the lexicographic order, so that most down links a site reads
 // (its z and y neighbours') are the up links its own block reads, and the
-// blocks are dealt out to the eight XCDs in contiguous ranges (t innermost
-// where the timeslices allow), so that the x and t neighbours' links are
-// still in that XCD's L2: each link comes from HBM about once.
+// blocks are dealt out to the eight XCDs in contiguous ranges, t innermost
+// (su3gf_order.h), so that the x and t neighbours' links are still in that
+// XCD's L2: each link comes from HBM about once.
 template <typename R, int S>
 __device__ __forceinline__ void load_site_link(const QualityArgs<R> &a, int64_t idx, int mu, M3<R> &u)
 {
@@ -271,31 +271,12 @@ __device__ __forceinline__ void quality_site(const QualityArgs<R> &a, int64_t si
     dGff = result;
 }
 
-// logical block of this block, or -1 for a block past the last one
-template <typename R> __device__ __forceinline__ int64_t quality_block(const QualityArgs<R> &a)
-{
-    const uint32_t b = blockIdx.x;
-    if (a.remap == 0) return b;
-    const uint32_t xcd = b & 7, k = b >> 3;
-    if (a.remap == 1) {
-        const int64_t per = (a.nblocks + 7) / 8;
-        const int64_t L = (int64_t)xcd * per + k;
-        return L < a.nblocks ? L : -1;
-    }
-    const uint32_t P = (uint32_t)a.tpass;
-    const uint32_t pass = fdiv(k, a.pass_div);
-    const uint32_t rem = k - pass * P * (uint32_t)a.slice_blocks;
-    const uint32_t q = fdiv(rem, a.tpass_div);
-    const int64_t t = (int64_t)xcd * a.slices_per_xcd + pass * P + (rem - q * P);
-    return t * a.slice_blocks + q;
-}
-
 constexpr int kQualitySites = 128;  // sites of each parity per block
 
 template <typename R, int G, int S>
 __global__ __launch_bounds__(kBlock) void k_quality(QualityArgs<R> a)
 {
-    const int64_t L = quality_block(a);
+    const int64_t L = ordered_block(a.order, blockIdx.x);
     const int par = threadIdx.x >= kQualitySites;
     const int64_t p = L * kQualitySites + (threadIdx.x & (kQualitySites - 1));
     const bool active = L >= 0 && p < a.g.Vh;
@@ -340,21 +321,8 @@ template <typename R, int S>
 static hipError_t launch_quality_s(int gauge, QualityArgs<R> a, hipStream_t s)
 {
     static_assert(2 * kQualitySites == kBlock, "a block holds both parities' sites");
-    a.nblocks = quality_blocks(a.g.V);
-    const int64_t half_slice = a.g.Vh / a.g.N[0];
-    unsigned grid;
-    if (a.g.N[0] % 8 == 0 && half_slice % kQualitySites == 0 && a.nblocks % 8 == 0) {
-        a.remap = 2;
-        a.slice_blocks = half_slice / kQualitySites;
-        a.slices_per_xcd = a.g.N[0] / 8;
-        if (a.tpass <= 0 || a.slices_per_xcd % a.tpass != 0) a.tpass = a.slices_per_xcd;
-        a.tpass_div = make_fastdiv((uint32_t)a.tpass);
-        a.pass_div = make_fastdiv((uint32_t)(a.tpass * a.slice_blocks));
-        grid = (unsigned)a.nblocks;
-    } else {
-        a.remap = 1;
-        grid = (unsigned)(8 * ((a.nblocks + 7) / 8));
-    }
+    a.order = make_block_order(quality_blocks(a.g.V), a.g.N[0], a.tpass);
+    const unsigned grid = (unsigned)order_grid(a.order);
     switch (gauge) {
     case GF_COULOMB: hipLaunchKernelGGL((k_quality<R, GF_COULOMB, S>), dim3(grid), dim3(kBlock), 0, s, a); break;
     case GF_MAG: hipLaunchKernelGGL((k_quality<R, GF_MAG, S>), dim3(grid), dim3(kBlock), 0, s, a); break;

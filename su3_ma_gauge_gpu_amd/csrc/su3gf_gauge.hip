@@ -143,6 +143,7 @@ __device__ __forceinline__ uint32_t tile_off(uint32_t boff, uint32_t words)
 // device scope, for g that a block on another XCD writes or reads within the
 // same launch (the pipelined sweep); 0 is the default policy.
 constexpr int kSc1 = 16;
+constexpr int kNt = 2;  // non-temporal: streamed past the caches (kept_link)
 
 // rows 0,1 of site byte offset boff
 template <typename A, int CP = 0> __device__ __forceinline__ void load_rows01(const Field &f, uint32_t boff, M3<A> &u)
@@ -172,14 +173,14 @@ template <typename A, int CP = 0> __device__ __forceinline__ void load_rows01(co
 constexpr double kQ24 = 8388607.0;  // 2^23 - 1: +-1 are exact
 constexpr float kInvQ24 = (float)(1.0 / kQ24);
 
-template <typename A> __device__ __forceinline__ void load_rows01_q24(const Field &f, uint32_t boff, M3<A> &u)
+template <typename A, int CP = 0> __device__ __forceinline__ void load_rows01_q24(const Field &f, uint32_t boff, M3<A> &u)
 {
     A v[12];
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        const uint32_t w0 = __builtin_amdgcn_raw_buffer_load_b32(f.r, (int)boff, (int)((3 * k) * f.V4), 0);
-        const uint32_t w1 = __builtin_amdgcn_raw_buffer_load_b32(f.r, (int)boff, (int)((3 * k + 1) * f.V4), 0);
-        const uint32_t w2 = __builtin_amdgcn_raw_buffer_load_b32(f.r, (int)boff, (int)((3 * k + 2) * f.V4), 0);
+        const uint32_t w0 = __builtin_amdgcn_raw_buffer_load_b32(f.r, (int)boff, (int)((3 * k) * f.V4), CP);
+        const uint32_t w1 = __builtin_amdgcn_raw_buffer_load_b32(f.r, (int)boff, (int)((3 * k + 1) * f.V4), CP);
+        const uint32_t w2 = __builtin_amdgcn_raw_buffer_load_b32(f.r, (int)boff, (int)((3 * k + 2) * f.V4), CP);
         // the bit-field builtin's result type is unsigned: convert it as the signed value it holds
         const int a = (int)__builtin_amdgcn_sbfe((int)w0, 0, 24);
         const int b = (int)__builtin_amdgcn_sbfe((int)__builtin_amdgcn_alignbit(w1, w0, 24), 0, 24);
@@ -211,7 +212,7 @@ __device__ __forceinline__ Field make_tiled_field64(const double *base, int64_t 
 }
 __device__ __forceinline__ uint32_t tile_off64(uint32_t boff) { return (boff & ~511u) * 12 + (boff & 511u); }
 
-template <typename A> __device__ __forceinline__ void load_rows01_64(const Field &f, uint32_t boff, M3<A> &u)
+template <typename A, int CP = 0> __device__ __forceinline__ void load_rows01_64(const Field &f, uint32_t boff, M3<A> &u)
 {
 #pragma unroll
     for (int i = 0; i < 2; i++)
@@ -219,9 +220,9 @@ template <typename A> __device__ __forceinline__ void load_rows01_64(const Field
         for (int j = 0; j < 3; j++) {
             const int comp = 2 * (j + 3 * i);
             const double re = __builtin_bit_cast(
-                double, __builtin_amdgcn_raw_buffer_load_b64(f.r, (int)boff, (int)(comp * f.V4), 0));
+                double, __builtin_amdgcn_raw_buffer_load_b64(f.r, (int)boff, (int)(comp * f.V4), CP));
             const double im = __builtin_bit_cast(
-                double, __builtin_amdgcn_raw_buffer_load_b64(f.r, (int)boff, (int)((comp + 1) * f.V4), 0));
+                double, __builtin_amdgcn_raw_buffer_load_b64(f.r, (int)boff, (int)((comp + 1) * f.V4), CP));
             u.e[i][j] = cx((A)re, (A)im);
         }
 }
@@ -231,11 +232,19 @@ template <int LF> __device__ __forceinline__ uint32_t site_boff(int64_t i) { ret
 
 // U0 rows 0,1 of the site at byte offset boff (site_boff): FP32 planes (LF =
 // 0), 24-bit fixed point in tiles (LF = 1) or FP64 in tiles (LF = 2)
-template <typename A, int LF> __device__ __forceinline__ void load_links(const Field &f, uint32_t boff, M3<A> &u)
+template <typename A, int LF, int CP = 0> __device__ __forceinline__ void load_links(const Field &f, uint32_t boff, M3<A> &u)
 {
-    if (LF == 2) load_rows01_64(f, tile_off64(boff), u);
-    else if (LF == 1) load_rows01_q24(f, tile_off(boff, 9), u);
-    else load_rows01(f, boff, u);
+    if (LF == 2) load_rows01_64<A, CP>(f, tile_off64(boff), u);
+    else if (LF == 1) load_rows01_q24<A, CP>(f, tile_off(boff, 9), u);
+    else load_rows01<A, CP>(f, boff, u);
+}
+
+// STREAM: the link kept in the caches or streamed past them (kept_link)
+template <typename A, int LF, bool STREAM>
+__device__ __forceinline__ void load_links(const Field &f, uint32_t boff, M3<A> &u, bool kept)
+{
+    if (STREAM && !kept) load_links<A, LF, kNt>(f, boff, u);
+    else load_links<A, LF>(f, boff, u);
 }
 
 // the field of U0_mu (one direction)
@@ -254,14 +263,14 @@ template <int LF, typename Args> __device__ __forceinline__ Field g_field(const 
 }
 template <typename A, int LF, int CP = 0> __device__ __forceinline__ void load_g(const Field &f, uint32_t boff, M3<A> &u)
 {
-    static_assert(LF != 2 || CP == 0, "FP64 g is only swept by the two kernels");
-    if (LF == 2) load_rows01_64(f, tile_off64(boff), u);
+    static_assert(LF != 2 || CP != kSc1, "FP64 g is only swept by the two kernels");
+    if (LF == 2) load_rows01_64<A, CP>(f, tile_off64(boff), u);
     else load_rows01<A, CP>(f, tile_off(boff, 12), u);
 }
 
 typedef unsigned int B64 __attribute__((__vector_size__(8)));  // the 64-bit buffer store's operand
 
-template <typename A> __device__ __forceinline__ void store_rows01_64(const Field &f, uint32_t boff, const M3<A> &u)
+template <typename A, int CP = 0> __device__ __forceinline__ void store_rows01_64(const Field &f, uint32_t boff, const M3<A> &u)
 {
 #pragma unroll
     for (int i = 0; i < 2; i++)
@@ -269,9 +278,9 @@ template <typename A> __device__ __forceinline__ void store_rows01_64(const Fiel
         for (int j = 0; j < 3; j++) {
             const int comp = 2 * (j + 3 * i);
             __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(B64, (double)u.e[i][j].x), f.r, (int)boff,
-                                                  (int)(comp * f.V4), 0);
+                                                  (int)(comp * f.V4), CP);
             __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(B64, (double)u.e[i][j].y), f.r, (int)boff,
-                                                  (int)((comp + 1) * f.V4), 0);
+                                                  (int)((comp + 1) * f.V4), CP);
         }
 }
 
@@ -289,11 +298,17 @@ template <typename A, int CP = 0> __device__ __forceinline__ void store_rows01(c
         }
 }
 
-template <typename A, int LF, int CP = 0> __device__ __forceinline__ void store_g(const Field &f, uint32_t boff, const M3<A> &u)
+// policy: 0, kNt, or (FP32 g) kSc1
+template <typename A, int LF> __device__ __forceinline__ void store_g(const Field &f, uint32_t boff, const M3<A> &u, int policy = 0)
 {
-    static_assert(LF != 2 || CP == 0, "FP64 g is only swept by the two kernels");
-    if (LF == 2) store_rows01_64(f, tile_off64(boff), u);
-    else store_rows01<A, CP>(f, tile_off(boff, 12), u);
+    if (LF == 2) {
+        if (policy == kNt) store_rows01_64<A, kNt>(f, tile_off64(boff), u);
+        else store_rows01_64(f, tile_off64(boff), u);
+    } else {
+        if (policy == kSc1) store_rows01<A, kSc1>(f, tile_off(boff, 12), u);
+        else if (policy == kNt) store_rows01<A, kNt>(f, tile_off(boff, 12), u);
+        else store_rows01(f, tile_off(boff, 12), u);
+    }
 }
 
 // Z = rows 0,1 of X Y^dagger (Y complete), then row 2 of the SU(3) product
@@ -450,32 +465,6 @@ template <typename A> __device__ __forceinline__ void theta_from_m(const M3<A> &
     theta_site<GF_LANDAU>(s, th, gf);
 }
 
-// Block order.  The eight XCDs take blocks round-robin (block b runs on XCD
-// b % 8), each with its own L2.  remap = 1 deals the blocks out so that each
-// XCD works through one contiguous eighth of the sites, which keeps the x, y
-// and z neighbours' g in that XCD's L2.  remap = 2 (Nt divisible by 8 and a
-// timeslice of one parity a whole number of 64-site blocks) also walks each
-// XCD's eighth -- Nt/8 timeslices -- with t innermost, so that the t
-// neighbours' g is read from L2 too: in plain order they are a timeslice
-// (V3/2 sites, megabytes of traffic) apart.  With t innermost, a block's x
-// neighbours are (blocks per timeslice row of x) x (timeslices walked
-// together) blocks away in the XCD's sequence; walking the XCD's timeslices in
-// passes of tpass shortens that distance (more x neighbours in L2) at the
-// cost of the t neighbours across a pass boundary.
-__device__ __forceinline__ int64_t logical_block(const GaugeSweepArgs &a)
-{
-    const uint32_t b = blockIdx.x, n = gridDim.x;  // below 2^31
-    if (a.remap == 0) return b;
-    const uint32_t xcd = b & 7, k = b >> 3;
-    if (a.remap == 1) return (int64_t)xcd * (n >> 3) + k;
-    const uint32_t P = (uint32_t)a.tpass;
-    const uint32_t pass = fdiv(k, a.pass_div);
-    const uint32_t rem = k - pass * P * (uint32_t)a.slice_blocks;
-    const uint32_t q = fdiv(rem, a.tpass_div);
-    const int64_t t = (int64_t)xcd * a.slices_per_xcd + pass * P + (rem - q * P);  // timeslice
-    return t * a.slice_blocks + q;
-}
-
 // Wavefront launch: the parity and logical block of this block, or false for
 // a padding block (uniform over the block)
 __device__ __forceinline__ bool wave_block(const GaugeSweepArgs &a, int64_t &blk, int &parity)
@@ -518,24 +507,29 @@ __device__ __forceinline__ void gauge_update(A q[4], float param, Philox &rng)
 
 // The direction-mu terms of site x (coordinates c, parity par):
 // X = U0_mu(x) g(y)^dagger and Z = g(z) U0_mu(z), y = x+mu, z = x-mu, so that
-// S_mu = X^dagger + Z.  coh (uniform): the neighbours' g through loads
-// coherent at device scope.
-template <typename A, int LF, typename Args>
-__device__ __forceinline__ void direction_terms(const Args &a, const Field &fg, int mu, const int c[4],
-                                                int par, uint32_t site_off, M3<A> &X, M3<A> &Z, bool coh = false)
+// S_mu = X^dagger + Z.  Each link is read once per half-sweep, g(y) and g(z)
+// by all of their neighbours.  STREAM: part of the links is streamed past the
+// caches, k the place of mu among the gauge's directions (kept_link).
+template <typename A, int LF, bool STREAM, typename Args>
+__device__ __forceinline__ void direction_terms(const Args &a, const Field &fg, int mu, int k, const int c[4], int par,
+                                                int64_t site, M3<A> &X, M3<A> &Z)
 {
     M3<A> T, W;
+    const int64_t z = backward(a.geo, c, par, mu);
     const uint32_t y_off = site_boff<LF>(forward(a.geo, c, par, mu));
-    const uint32_t z_off = site_boff<LF>(backward(a.geo, c, par, mu));
+    const uint32_t z_off = site_boff<LF>(z);
     const Field fu = links_field<LF>(a.U0, a.geo.V, mu);
-    load_links<A, LF>(fu, site_off, W);
-    if (LF != 2 && coh) load_g<A, LF, LF == 2 ? 0 : kSc1>(fg, y_off, T);
-    else load_g<A, LF>(fg, y_off, T);
+    bool kx = true, kz = true;
+    if constexpr (STREAM) {
+        kx = kept_link(a.keep, a.geo.Vh, par ? site - a.geo.Vh : site, k);
+        kz = kept_link(a.keep, a.geo.Vh, par ? z : z - a.geo.Vh, k);
+    }
+    load_links<A, LF, STREAM>(fu, site_boff<LF>(site), W, kx);
+    load_g<A, LF>(fg, y_off, T);
     third_row(T);
     prod_adag(X, W, T);  // U0_mu(x) g(y)^dagger
-    if (LF != 2 && coh) load_g<A, LF, LF == 2 ? 0 : kSc1>(fg, z_off, T);
-    else load_g<A, LF>(fg, z_off, T);
-    load_links<A, LF>(fu, z_off, W);
+    load_g<A, LF>(fg, z_off, T);
+    load_links<A, LF, STREAM>(fu, z_off, W, kz);
     third_row(W);
     prod_ab(Z, T, W);  // g(z) U0_mu(z)
 }
@@ -547,7 +541,7 @@ __device__ __forceinline__ void direction_terms(const Args &a, const Field &fg, 
 template <typename A, int G, int ALGO, int THETA, int LF, typename SumS, typename Args>
 __device__ __forceinline__ void site_tail(const Args &a, const Field &fg, uint32_t site_off, bool active,
                                           int64_t blk, int lane, const SumS &sum_s, M3<A> Gx, Philox &rng,
-                                          bool sc1_store = false)
+                                          int store_policy = 0)
 {
     static_assert(THETA == 0 || ALGO != GF_RANDOM, "the random transformation forms no S to check");
     third_row(Gx);
@@ -600,10 +594,7 @@ __device__ __forceinline__ void site_tail(const Args &a, const Field &fg, uint32
     }
 
     project_rows01(Gx);  // keep g unitary at the precision it is stored in
-    if (active) {
-        if (LF != 2 && sc1_store) store_g<A, LF, LF == 2 ? 0 : kSc1>(fg, site_off, Gx);
-        else store_g<A, LF>(fg, site_off, Gx);
-    }
+    if (active) store_g<A, LF>(fg, site_off, Gx, store_policy);
 
     if (THETA == 2 && active) {  // the state after the update, with g(x) as stored
         third_row(Gx);
@@ -638,7 +629,7 @@ template <typename Args> __device__ __forceinline__ void site_rng(const Args &a,
 // LDS; wave 0 adds them in the order of mu and runs the tail.  gsweep_block
 // sweeps the sites of parity `parity` in the 64-site block blk of the lattice
 // of a; k_gsweep and k_gsweep_multi choose the block.
-template <typename A, int G, int ALGO, int THETA, int LF, typename Args>
+template <typename A, int G, int ALGO, int THETA, int LF, bool STREAM, typename Args>
 __device__ __forceinline__ void gsweep_block(const Args &a, int64_t blk, int parity)
 {
     constexpr int kW = gsweep_waves<G>();
@@ -654,8 +645,14 @@ __device__ __forceinline__ void gsweep_block(const Args &a, int64_t blk, int par
     const uint32_t site_off = site_boff<LF>(site);
     const Field fg = g_field<LF>(a);
 
+    // the sites' own g, read and written here alone
+    bool stream_g = false;
+    if constexpr (STREAM) stream_g = a.stream_g;
     M3<A> Gx;
-    if (wave == 0) load_g<A, LF>(fg, site_off, Gx);
+    if (wave == 0) {
+        if (stream_g) load_g<A, LF, kNt>(fg, site_off, Gx);
+        else load_g<A, LF>(fg, site_off, Gx);
+    }
 
     Philox rng;
     if (ALGO == GF_SA || ALGO == GF_RANDOM) site_rng(a, p, parity, rng);
@@ -665,7 +662,7 @@ __device__ __forceinline__ void gsweep_block(const Args &a, int64_t blk, int par
         if (wave != 0) return;
     } else {
         M3<A> X, Z;
-        direction_terms<A, LF>(a, fg, mu, c, par, site_off, X, Z);
+        direction_terms<A, LF, STREAM>(a, fg, mu, wave, c, par, site, X, Z);
 #pragma unroll
         for (int i = 0; i < 3; i++)
 #pragma unroll
@@ -696,10 +693,10 @@ __device__ __forceinline__ void gsweep_block(const Args &a, int64_t blk, int par
                 S.e[i][j] = cx(v[0], v[1]);
             }
     };
-    site_tail<A, G, ALGO, THETA, LF>(a, fg, site_off, active, blk, lane, sum_s, Gx, rng);
+    site_tail<A, G, ALGO, THETA, LF>(a, fg, site_off, active, blk, lane, sum_s, Gx, rng, stream_g ? kNt : 0);
 }
 
-template <typename A, int G, int ALGO, int THETA, int LF>
+template <typename A, int G, int ALGO, int THETA, int LF, bool STREAM>
 __global__ __launch_bounds__(kGBlock) void k_gsweep(GaugeSweepArgs a)
 {
     static_assert(LF != 2 || sizeof(A) == 8, "FP64 storage takes FP64 arithmetic");
@@ -710,15 +707,15 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep(GaugeSweepArgs a)
     if (a.wf) {
         if (!wave_block(a, blk, parity)) return;
     } else {
-        blk = logical_block(a);
+        blk = ordered_block(a.order, blockIdx.x);
+        if (blk < 0) return;
     }
-    gsweep_block<A, G, ALGO, THETA, LF>(a, blk, parity);
+    gsweep_block<A, G, ALGO, THETA, LF, STREAM>(a, blk, parity);
 }
 
 // Several lattices in one launch (the annealing of a batch): their blocks of
 // one parity are concatenated in lattice order, and the XCDs take contiguous
-// eighths of that sequence (block b runs on XCD b % 8), as remap = 1 does for
-// one lattice.  Lattice k's sites are those of the single-lattice sweep with
+// eighths of that sequence (block b runs on XCD b % 8).  Lattice k's sites are those of the single-lattice sweep with
 // its own seed and RNG counter item[k].counter + counter_add + parity: the
 // same updates and random numbers.  The lattice's fields as gsweep_block reads
 // them, its geometry by reference into the kernel argument (indexed by
@@ -746,7 +743,7 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_multi(MultiSweepArgs m)
     const MultiItem &it = m.item[k];
     const MultiView a{it.U0, it.g, it.geo, m.param, it.seed, it.counter + m.counter_add + (uint32_t)m.parity,
                       32, 0, 0, nullptr};
-    gsweep_block<A, G, ALGO, 0, LF>(a, L - m.first[k], m.parity);
+    gsweep_block<A, G, ALGO, 0, LF, false>(a, L - m.first[k], m.parity);
 }
 
 // ------------------------------------------------------ pipelined sweep
@@ -955,7 +952,7 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_pipe(GaugeSweepArgs a)
             }
     };
     // even sites: g stored coherently at device scope (read by odd items of this launch)
-    site_tail<A, G, ALGO, 0, LF>(a, fg, site_off, active, blk, lane, sum_s, Gx, rng, !odd);
+    site_tail<A, G, ALGO, 0, LF>(a, fg, site_off, active, blk, lane, sum_s, Gx, rng, odd ? 0 : kSc1);
     if (odd) return;
     // the stores are complete before the flag says so
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -980,7 +977,7 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_pipe(GaugeSweepArgs a)
 // inverse square roots.  Wave 0 also updates and stores g(x).
 // theta (THETA = 1 before, 2 after the update) comes from the links as in the
 // link sweep's MAG check.
-template <typename A, int ALGO, int THETA, int LF>
+template <typename A, int ALGO, int THETA, int LF, bool STREAM>
 __global__ __launch_bounds__(kGBlock) void k_gsweep_mag(GaugeSweepArgs a)
 {
     constexpr int kX = 4 * 3 * 64;  // one exchange: [direction 4][D, Im c, Re c][lane 64]
@@ -997,7 +994,8 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_mag(GaugeSweepArgs a)
     if (a.wf) {
         if (!wave_block(a, blk, parity)) return;
     } else {
-        blk = logical_block(a);
+        blk = ordered_block(a.order, blockIdx.x);
+        if (blk < 0) return;
     }
     bool active;
     const int64_t p = block_site(a.geo, blk, lane, active);
@@ -1016,7 +1014,7 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_mag(GaugeSweepArgs a)
     M3<A> up, dn;
     {
         M3<A> X, Z;
-        direction_terms<A, LF>(a, fg, mu, c, par, site_off, X, Z);
+        direction_terms<A, LF, STREAM>(a, fg, mu, mu, c, par, site, X, Z);
         prod_ab(up, Gx, X);    // g(x) U0_mu(x) g(y)^dagger
         prod_adag(dn, Z, Gx);  // g(z) U0_mu(z) g(x)^dagger
     }
@@ -1116,14 +1114,19 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_mag(GaugeSweepArgs a)
 // blocks of a launch: one per logical block, or a wavefront launch's even and odd grids
 inline int64_t gsweep_grid(const GaugeSweepArgs &a)
 {
-    if (!a.wf) return sweep_grid(a.geo);
+    if (!a.wf) return order_grid(a.order);
     return a.wf_even_grid + 8 * ((a.wf_odd_n + a.wf_odd1_n + 7) / 8);
 }
+
+// A wavefront launch keeps every link cached: its odd update of a timeslice
+// reads the links that the even one before it brought in.
+inline bool gsweep_streams(const GaugeSweepArgs &a) { return !a.wf && a.keep < 4 * a.geo.Vh; }
 
 template <typename A, int ALGO, int THETA, int LF> void launch_k_mag(const GaugeSweepArgs &a, hipStream_t s)
 {
     const dim3 grid((unsigned)gsweep_grid(a)), block(kGBlock);
-    hipLaunchKernelGGL((k_gsweep_mag<A, ALGO, THETA, LF>), grid, block, 0, s, a);
+    if (gsweep_streams(a)) hipLaunchKernelGGL((k_gsweep_mag<A, ALGO, THETA, LF, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((k_gsweep_mag<A, ALGO, THETA, LF, false>), grid, block, 0, s, a);
 }
 
 template <typename A, int LF> hipError_t launch_mag_lf(int algo, int theta, const GaugeSweepArgs &a, hipStream_t s)
@@ -1166,7 +1169,8 @@ template <typename A, int G, int ALGO, int THETA, int LF>
 void launch_k(const GaugeSweepArgs &a, hipStream_t s)
 {
     const dim3 grid((unsigned)gsweep_grid(a)), block(64 * gsweep_waves<G>());
-    hipLaunchKernelGGL((k_gsweep<A, G, ALGO, THETA, LF>), grid, block, 0, s, a);
+    if (gsweep_streams(a)) hipLaunchKernelGGL((k_gsweep<A, G, ALGO, THETA, LF, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((k_gsweep<A, G, ALGO, THETA, LF, false>), grid, block, 0, s, a);
 }
 
 template <typename A, int G> hipError_t launch_g(int algo, int theta, const GaugeSweepArgs &a, hipStream_t s)
@@ -1304,25 +1308,35 @@ hipError_t launch_pack24(int ti, int si, const void *U, uint32_t *P, int64_t V, 
     return hipGetLastError();
 }
 
+namespace {
+// What the two-kernel sweep keeps in the Infinity Cache: g, which every
+// neighbour reads again, and of the links what g leaves room for (24-bit
+// links at 36^4: 91 us per launch with everything cached, 64 us keeping 131
+// MB of them; FP64 at 32^4: 107 and 90 us keeping 160 MB; 24-bit at 48^4, no
+// room: 246 and 209 us).  Where g alone is larger than the cache, a site's own
+// g, which the half-sweep reads and writes once, is streamed as well (FP64 at
+// 44^4: 415 us and 390, at 48^4: 581 and 547; at 40^4, where g fits, 241 us
+// became 251).
+void cache_policy(int gauge, GaugeSweepArgs &a)
+{
+    const int dirs = gauge == GF_COULOMB ? 3 : 4;
+    const int64_t V = a.geo.V, g = 12 * (a.links64 ? 8 : 4) * V;
+    const int64_t links = dirs * (a.links64 ? 96 : a.links24 ? 36 : 48) * V;
+    a.stream_g = g > kInfinityCacheBytes;
+    a.keep = 4 * a.geo.Vh;
+    if (links + g > kInfinityCacheBytes)
+        a.keep = g < kKeptBytes ? (int64_t)((double)(dirs * a.geo.Vh) * (double)(kKeptBytes - g) / (double)links) : 0;
+}
+}  // namespace
+
 hipError_t launch_gsweep(int gauge, int algo, int theta, bool fp64_arith, const GaugeSweepArgs &a, hipStream_t s)
 {
     if (!gauge_sweep_fits(a.geo.V)) return hipErrorInvalidValue;
     if (a.links64 && (!fp64_arith || !gauge_sweep64_fits(a.geo.V))) return hipErrorInvalidValue;
     if (theta == 3 && !a.state) return hipErrorInvalidValue;
     GaugeSweepArgs b = a;
-    const int64_t half_slice = a.geo.Vh / a.geo.N[0];  // sites of one parity in a timeslice
-    if (b.remap && a.geo.N[0] % 8 == 0 && half_slice % 64 == 0) {
-        b.remap = 2;
-        b.slice_blocks = half_slice / 64;
-        b.slices_per_xcd = a.geo.N[0] / 8;
-        if (b.tpass <= 0 || b.slices_per_xcd % b.tpass != 0) b.tpass = b.slices_per_xcd;
-        b.tpass_div = make_fastdiv((uint32_t)b.tpass);
-        b.pass_div = make_fastdiv((uint32_t)(b.tpass * b.slice_blocks));
-    } else if (b.remap && sweep_grid(a.geo) % 8 == 0) {
-        b.remap = 1;
-    } else {
-        b.remap = 0;
-    }
+    b.order = make_block_order(sweep_grid(a.geo), a.geo.N[0], a.tpass);
+    cache_policy(gauge, b);
     if (b.nsb <= 0) b.nsb = 32;
     b.wf = 0;
     return fp64_arith ? launch_a<double>(gauge, algo, theta, b, s) : launch_a<float>(gauge, algo, theta, b, s);
@@ -1421,7 +1435,6 @@ hipError_t launch_gsweep_pipe(int gauge, int algo, bool fp64_arith, const GaugeS
     b.pipe_launch = ++*a.pipe_count;
     b.pipe_tdiv = make_fastdiv((uint32_t)b.plan.T);
     b.wf = 0;
-    b.remap = 0;
     if (b.nsb <= 0) b.nsb = 32;
     const hipError_t e = gauge == GF_LANDAU    ? launch_pipe_lf<GF_LANDAU>(algo, fp64_arith, b, s)
                          : gauge == GF_COULOMB ? launch_pipe_lf<GF_COULOMB>(algo, fp64_arith, b, s)

@@ -82,15 +82,11 @@ template <typename R> struct QualityArgs {
     double *dGff, *dA;  // optional per-site outputs (V doubles each)
     double *partial;    // optional per-block (theta, gff) partials
     int crit_max;
-    // block order, set by the launcher: a block takes the sites of both
-    // parities with parity-split index in [128 L, 128 L + 128) (256
-    // consecutive sites of the lexicographic order) for its logical block L
-    int remap;              // 0 plain, 1 one contiguous eighth per XCD, 2 the same with t innermost
-    int64_t nblocks;        // logical blocks (quality_blocks)
-    int64_t slice_blocks;   // remap 2: logical blocks per timeslice
-    int slices_per_xcd;     // remap 2
-    int tpass;              // remap 2: each XCD's timeslices walked in passes of tpass (0: one pass)
-    FastDiv tpass_div, pass_div;  // division by tpass and by tpass * slice_blocks
+    // a block takes the sites of both parities with parity-split index in
+    // [128 L, 128 L + 128) (256 consecutive sites of the lexicographic order)
+    // for its logical block L
+    int tpass;         // the block order's span: timeslices walked together, t innermost (order_span)
+    BlockOrder order;  // set by the launcher
 };
 
 
@@ -104,12 +100,11 @@ struct GaugeSweepArgs {
     Geom geo;
     int parity;
     float param;       // OR parameter or SA temperature
-    int remap;         // block order: 0 plain, else chosen by the launcher (XCD-aware)
-    int slices_per_xcd;  // set by the launcher for remap = 2
-    int64_t slice_blocks;
-    int tpass;           // remap = 2: each XCD walks its timeslices in passes of tpass (a divisor of
-                         // slices_per_xcd; 0 = all of them in one pass), t innermost within a pass
-    FastDiv tpass_div, pass_div;  // division by tpass and by tpass * slice_blocks
+    int tpass;         // the block order's span: timeslices walked together, t innermost (order_span)
+    BlockOrder order;  // set by the launcher
+    int64_t keep;      // set by the launcher: the links of each parity kept in the Infinity Cache
+                       // (kept_link); the two-kernel sweep streams the others
+    bool stream_g;     // set by the launcher: the updated sites' own g is streamed too
     uint32_t seed, counter;  // SA / random transformation (Philox key and counter)
     int64_t nsb;       // sites per block of the reference launch (RNG key)
     int links24;       // U0 in the 24-bit fixed-point form of launch_pack24 (OR, SA, microcanonical)
