@@ -355,6 +355,15 @@ __device__ __forceinline__ void philox_init(Philox &p, uint32_t tid, uint32_t se
     p.local = 0;
 }
 
+// key word 0 of site p of a parity: the global id of the reference's thread of
+// that site (mu = 0, up) in its launch of V/2/nsb x 8 nsb threads
+// (PhiloxWrapper.hxx:93-110)
+__device__ __forceinline__ uint32_t rng_tid(int64_t p, int64_t nsb)
+{
+    const uint32_t n = (uint32_t)p, b = (uint32_t)nsb;  // p < 2^31
+    return n / b * 8 * b + n % b;
+}
+
 __device__ __forceinline__ void philox_block(Philox &p)
 {
     p.c0++;
@@ -391,6 +400,59 @@ __device__ __forceinline__ float philox_rand(Philox &p, float)
     p.w2 = p.w1;
     p.w1 = p.w0;
     return (float)(1 + (p.w3 >> 8)) * 0x1.fffffep-25f;
+}
+
+// Draws per Philox block of a uniform of type RAND, and the number of draws
+// handed out so far.
+template <typename RAND> constexpr uint32_t draws_per_block() { return sizeof(RAND) == 8 ? 2 : 4; }
+template <typename RAND> __device__ __forceinline__ uint32_t philox_pos(const Philox &p)
+{
+    return draws_per_block<RAND>() * p.c0 - (uint32_t)p.local;
+}
+
+// the generator after `pos` draws
+template <typename RAND> __device__ __forceinline__ void philox_seek(Philox &p, uint32_t pos)
+{
+    p.c0 = pos / draws_per_block<RAND>();
+    p.local = 0;
+    const uint32_t skip = pos % draws_per_block<RAND>();
+    if (skip > 0) (void)philox_rand(p, RAND(0));
+    if (skip > 1) (void)philox_rand(p, RAND(0));
+    if (skip > 2) (void)philox_rand(p, RAND(0));
+}
+
+// draws pos, pos + 1, pos + 2, pos + 3 of the stream of key (k0, k1) and launch
+// counter c1: what four calls of philox_rand return after `pos` draws
+__device__ __forceinline__ void philox_at(uint32_t k0, uint32_t k1, uint32_t c1, uint32_t pos, double u[4])
+{
+    Philox p;
+    p.k0 = k0;
+    p.k1 = k1;
+    p.c1 = c1;
+    philox_seek<double>(p, pos);
+#pragma unroll
+    for (int k = 0; k < 4; k++) u[k] = philox_rand(p, 0.0);
+}
+__device__ __forceinline__ void philox_at(uint32_t k0, uint32_t k1, uint32_t c1, uint32_t pos, float u[4])
+{
+    uint32_t a[4] = {pos / 4 + 1, c1, 0x12345678u, 0xabcdef09u}, b[4] = {0, 0, 0, 0};
+    philox10(a, k0, k1);
+    const uint32_t off = pos % 4;
+    if (off) {
+        b[0] = pos / 4 + 2;
+        b[1] = c1;
+        b[2] = 0x12345678u;
+        b[3] = 0xabcdef09u;
+        philox10(b, k0, k1);
+    }
+    // word w of the two blocks' draws, in the order they are handed out
+    const uint32_t s0 = a[3], s1 = a[2], s2 = a[1], s3 = a[0], s4 = b[3], s5 = b[2], s6 = b[1];
+    const uint32_t w[4] = {off == 0 ? s0 : off == 1 ? s1 : off == 2 ? s2 : s3,
+                           off == 0 ? s1 : off == 1 ? s2 : off == 2 ? s3 : s4,
+                           off == 0 ? s2 : off == 1 ? s3 : off == 2 ? s4 : s5,
+                           off == 0 ? s3 : off == 1 ? s4 : off == 2 ? s5 : s6};
+#pragma unroll
+    for (int k = 0; k < 4; k++) u[k] = (float)(1 + (w[k] >> 8)) * 0x1.fffffep-25f;
 }
 
 // ------------------------------------------------------ quad reductions

@@ -16,14 +16,169 @@ namespace exact {
 static inline unsigned blocks_for(int64_t threads) { return (unsigned)((threads + kBlock - 1) / kBlock); }
 
 // ------------------------------------------------------------------- sweep
-template <typename R, int G, int A, int S>
-static hipError_t launch_t(SweepArgs<R> a, hipStream_t s)
+// The half-sweep with an update that draws random numbers (heatbath,
+// stochastic relaxation, random transformation): k_sweep's mapping, but one
+// wave of the block makes the update and hands the SU(2) element to the
+// others through LDS (two barriers per subgroup, the same values).  In
+// k_sweep every wave computes its sites' update from the shared sums; a
+// heatbath costs more than the rest of the kernel, so that made four waves
+// repeat it, and its registers on top of the links' left 2 waves per SIMD in
+// FP64 (198 VGPRs).  PARK: the updating wave puts its links aside in LDS
+// meanwhile, which leaves 122 VGPRs and 4 waves per SIMD.  Heatbath half-sweep, Landau
+// at T = 0.3: FP64 32^4 250 -> 175 us, 24^4 95 -> 67; FP32 32^4 129 -> 92,
+// with the update in double 186 -> 118; MAG at T = 0.8, FP64 32^4 313 -> 186.
+// A fifth wave for the update, without links, needs no such copy but leaves
+// room for fewer blocks (FP64 Landau 32^4: 263 us).
+template <typename R, int G, int A, int S, bool STREAM, bool PARK>
+__global__ __launch_bounds__(kBlock) void k_sweep_rng(SweepArgs<R> a)
 {
-    const dim3 grid((unsigned)sweep_grid(a.g)), block(kBlock);
-    a.keep = kept_links(a.g.Vh, 48 * (int64_t)sizeof(R) * a.g.V);
-    if (a.keep < 4 * a.g.Vh) hipLaunchKernelGGL((k_sweep<R, G, A, S, true, 0, false, true>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((k_sweep<R, G, A, S, true, 0, false, false>), grid, block, 0, s, a);
+    constexpr bool kSums = A != GF_RANDOM;  // the random transformation does not read the links
+    constexpr int kQ = 4 * 64;              // an SU(2) element: [comp 4][lane 64]
+    constexpr int kX = 8 * 4 * 64;          // the links' contributions: [link 8][comp 4][lane 64]
+    __shared__ R lds[kSums ? kQ + kX + (PARK ? 36 * 64 : 0) : 3 * kQ];
+    R *const lx = lds + kQ, *const park = lds + kQ + kX;
+    const int mu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    // consecutive blocks of an XCD update with different waves, so that the
+    // updates of a CU's blocks are spread over its SIMDs
+    const bool updates = mu == (int)((blockIdx.x >> 3) & 3);
+    bool active;
+    const int64_t p = block_site(a.g, blockIdx.x, lane, active);
+    const int64_t site = (active ? p : 0) + (a.parity ? a.g.Vh : 0);
+    int c[4], par;
+    site_coords(a.g, site, c, par);
+    // Coulomb: as in k_sweep
+    const bool slice_dw = G == GF_COULOMB && mu == 0 && a.g.N[0] == 1;
+    const int64_t nb = slice_dw ? site : backward(a.g, c, par, mu);
+    const LinkRef<R> lu = link_ref(a.U, a.g.V, S, site, mu);
+    const LinkRef<R> ld = link_ref(slice_dw ? a.Udw : a.U, a.g.V, S, nb, mu);
+    const bool keep_up = !STREAM || kept_link(a.keep, a.g.Vh, active ? p : 0, mu);
+    const bool keep_dn = !STREAM || kept_link(a.keep, a.g.Vh, nb >= a.g.Vh ? nb - a.g.Vh : nb, mu);
+
+    Philox rng;
+    philox_init(rng, rng_tid(p, a.nsb), a.seed, a.counter);
+    if (!kSums && updates) {
+#pragma unroll 1
+        for (int sub = 0; sub < 3; sub++) {
+            const R none[8][4] = {};
+            R q[4];
+            site_update<R, G, A, true>(none, q, a.param, rng);
+#pragma unroll
+            for (int k = 0; k < 4; k++) lds[sub * kQ + k * 64 + lane] = q[k];
+        }
+    }
+
+    M3<R> up, dn;
+    if (active) {
+        if constexpr (STREAM) {
+            load12(lu, up, keep_up);
+            load12(ld, dn, keep_dn);
+        } else {
+            load12(lu, up);
+            load12(ld, dn);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = 0; j < 3; j++) { up.e[i][j] = cx((R)(i == j), (R)0); dn.e[i][j] = up.e[i][j]; }
+    }
+    reconstruct_e<true>(up);
+    reconstruct_e<true>(dn);
+    if (!kSums) __syncthreads();
+
+    auto subgroup = [&](auto I_, auto J_, int sub) {
+        constexpr int I = decltype(I_)::value, J = decltype(J_)::value;
+        R q[4];
+        if (kSums) {
+            R vu[4], vd[4];
+            link_contrib<R, G, I, J, true>(up, vu);
+            link_contrib<R, G, I, J, false>(dn, vd);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                lx[((0 + mu) * 4 + k) * 64 + lane] = vu[k];
+                lx[((4 + mu) * 4 + k) * 64 + lane] = vd[k];
+            }
+            __syncthreads();
+            if (updates) {
+                if constexpr (PARK) {
+#pragma unroll
+                    for (int k = 0; k < 9; k++) {
+                        const Cx<R> u = up.e[k / 3][k % 3], d = dn.e[k / 3][k % 3];
+                        R *const b = park + 4 * k * 64 + lane;
+                        b[0] = u.x; b[64] = u.y; b[128] = d.x; b[192] = d.y;
+                    }
+                    asm volatile("" ::: "memory");  // the links' registers are free until they come back
+                }
+                R cc[8][4];
+#pragma unroll
+                for (int m = 0; m < 8; m++)
+#pragma unroll
+                    for (int k = 0; k < 4; k++) cc[m][k] = lx[(m * 4 + k) * 64 + lane];
+                site_update<R, G, A, true>(cc, q, a.param, rng);
+#pragma unroll
+                for (int k = 0; k < 4; k++) lds[k * 64 + lane] = q[k];
+                if constexpr (PARK) {
+                    asm volatile("" ::: "memory");
+#pragma unroll
+                    for (int k = 0; k < 9; k++) {
+                        const R *const b = park + 4 * k * 64 + lane;
+                        up.e[k / 3][k % 3] = cx(b[0], b[64]);
+                        dn.e[k / 3][k % 3] = cx(b[128], b[192]);
+                    }
+                }
+            }
+            // the next writes to the exchange follow this barrier, after which
+            // the update has read it; the next element is written after the
+            // next exchange's barrier, past every wave's reads of this one
+            __syncthreads();
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) q[k] = lds[(kSums ? 0 : sub * kQ) + k * 64 + lane];
+        left_mult<R, I, J>(up, q);
+        right_mult_dag<R, I, J>(dn, q);
+    };
+    subgroup(std::integral_constant<int, 0>(), std::integral_constant<int, 2>(), 0);
+    subgroup(std::integral_constant<int, 1>(), std::integral_constant<int, 2>(), 1);
+    subgroup(std::integral_constant<int, 0>(), std::integral_constant<int, 1>(), 2);
+    if (active) {
+        if constexpr (STREAM) {
+            store12(lu, up, keep_up);
+            store12(ld, dn, keep_dn);
+        } else {
+            store12(lu, up);
+            store12(ld, dn);
+        }
+    }
+}
+
+// Up to two blocks per CU the registers are there in any case (PARK = false
+// leaves 2 waves per SIMD in FP64) and the copies only lengthen the update.
+// FP64 heatbath half-sweep with the links kept in registers and put aside, and
+// with every wave making the update as in k_sweep: Coulomb timeslice 32^3 (256
+// blocks) 15.6, 16.7 and 16.0 us, Landau 16^4 (512) 20.1, 21.3 and 23.3, 20^4
+// (1250) 44.6, 36.6 and 48.6.
+constexpr unsigned kUnparkedBlocks = 512;
+
+template <typename R, int G, int A, int S, bool STREAM> static hipError_t launch_s(const SweepArgs<R> &a, hipStream_t s)
+{
+    constexpr int AB = A % kDpUpdate;  // the update rule without its precision
+    const dim3 grid((unsigned)sweep_grid(a.g));
+    if constexpr (AB == GF_OR || AB == GF_MICRO)
+        hipLaunchKernelGGL((k_sweep<R, G, A, S, true, 0, false, STREAM>), grid, dim3(kBlock), 0, s, a);
+    else if constexpr (AB == GF_RANDOM)
+        hipLaunchKernelGGL((k_sweep_rng<R, G, A, S, STREAM, false>), grid, dim3(kBlock), 0, s, a);
+    else if (STREAM || grid.x > kUnparkedBlocks)
+        hipLaunchKernelGGL((k_sweep_rng<R, G, A, S, STREAM, true>), grid, dim3(kBlock), 0, s, a);
+    else if constexpr (!STREAM)
+        hipLaunchKernelGGL((k_sweep_rng<R, G, A, S, STREAM, false>), grid, dim3(kBlock), 0, s, a);
     return hipGetLastError();
+}
+
+template <typename R, int G, int A, int S> static hipError_t launch_t(SweepArgs<R> a, hipStream_t s)
+{
+    a.keep = kept_links(a.g.Vh, 48 * (int64_t)sizeof(R) * a.g.V);
+    return a.keep < 4 * a.g.Vh ? launch_s<R, G, A, S, true>(a, s) : launch_s<R, G, A, S, false>(a, s);
 }
 
 template <typename R, int G, int S>

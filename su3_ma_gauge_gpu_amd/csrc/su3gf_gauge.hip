@@ -534,16 +534,38 @@ __device__ __forceinline__ void direction_terms(const Args &a, const Field &fg, 
     prod_ab(Z, T, W);  // g(z) U0_mu(z)
 }
 
+// The heatbath needs as many registers as the matrices it works between; put
+// aside in LDS meanwhile (park: 9 complex numbers per matrix and lane), they
+// leave the heatbath sweep its occupancy: 70 VGPRs and 7 waves per SIMD
+// instead of 131 and 3.  One temperature (heatbath and three microcanonical
+// sweeps) at 32^4 on 24-bit links: 372 us, 389 us with them in registers.
+// (MAG's heatbath keeps its links in registers: put aside, the compiler rounds
+// their rotations differently, and it gains nothing.)
+template <typename A> __device__ __forceinline__ void put_aside(A *park, int lane, const M3<A> &m)
+{
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        park[(2 * k) * 64 + lane] = m.e[k / 3][k % 3].x;
+        park[(2 * k + 1) * 64 + lane] = m.e[k / 3][k % 3].y;
+    }
+}
+template <typename A> __device__ __forceinline__ void take_back(const A *park, int lane, M3<A> &m)
+{
+#pragma unroll
+    for (int k = 0; k < 9; k++) m.e[k / 3][k % 3] = cx(park[(2 * k) * 64 + lane], park[(2 * k + 1) * 64 + lane]);
+}
+constexpr int kParked = 18 * 64;  // reals of a matrix put aside by a wave
+
 // Given S = sum_mu g(y) U0_mu(x)^dagger + g(z) U0_mu(z) (from sum_s, which
 // reads it again for the theta of the updated state) and g(x) rows 0,1 in
 // Gx: the three subgroup updates of g(x), its store, and the fused-check
-// partial sums of the 64-site block blk.
+// partial sums of the 64-site block blk.  park: LDS that sum_s no longer needs
+// when only the update is left (2 kParked reals; the heatbath).
 template <typename A, int G, int ALGO, int THETA, int LF, typename SumS, typename Args>
 __device__ __forceinline__ void site_tail(const Args &a, const Field &fg, uint32_t site_off, bool active,
                                           int64_t blk, int lane, const SumS &sum_s, M3<A> Gx, Philox &rng,
-                                          int store_policy = 0)
+                                          A *park, int store_policy = 0)
 {
-    static_assert(THETA == 0 || ALGO != GF_RANDOM, "the random transformation forms no S to check");
     third_row(Gx);
 
     double th = 0, gf = 0;
@@ -551,7 +573,7 @@ __device__ __forceinline__ void site_tail(const Args &a, const Field &fg, uint32
     // they need and update only the entries a later step reads
     M3<A> M;
     zero(M);
-    if (ALGO != GF_RANDOM) {
+    {
         M3<A> S;
         sum_s(S);
         mac_adag(M, S, Gx);
@@ -566,10 +588,23 @@ __device__ __forceinline__ void site_tail(const Args &a, const Field &fg, uint32
         }
         return;
     }
+    const auto update = [&](A q[4]) {
+        if constexpr (ALGO == GF_SA) {
+            put_aside(park, lane, M);
+            put_aside(park + kParked, lane, Gx);
+            asm volatile("" ::: "memory");  // their registers are free until they come back
+            gauge_update<A, G, ALGO>(q, a.param, rng);
+            asm volatile("" ::: "memory");
+            take_back(park, lane, M);
+            take_back(park + kParked, lane, Gx);
+        } else {
+            gauge_update<A, G, ALGO>(q, a.param, rng);
+        }
+    };
     {   // subgroup (0,2): reads M00 M02 M20 M22; M00 M10 M02 M12 M22 are read later
         A q[4];
         quat<A, 0, 2>(M, q);
-        gauge_update<A, G, ALGO>(q, a.param, rng);
+        update(q);
         const Hd<A> h = su2_dag(q);
         const Cx<A> m00 = col_i(h, M.e[0][0], M.e[0][2]), m10 = col_i(h, M.e[1][0], M.e[1][2]);
         const Cx<A> m02 = col_j(h, M.e[0][0], M.e[0][2]), m12 = col_j(h, M.e[1][0], M.e[1][2]);
@@ -580,7 +615,7 @@ __device__ __forceinline__ void site_tail(const Args &a, const Field &fg, uint32
     {   // subgroup (1,2): reads M11 M12 M21 M22; M01 M11 are read later
         A q[4];
         quat<A, 1, 2>(M, q);
-        gauge_update<A, G, ALGO>(q, a.param, rng);
+        update(q);
         const Hd<A> h = su2_dag(q);
         const Cx<A> m01 = col_i(h, M.e[0][1], M.e[0][2]), m11 = col_i(h, M.e[1][1], M.e[1][2]);
         M.e[0][1] = m01; M.e[1][1] = m11;
@@ -589,7 +624,7 @@ __device__ __forceinline__ void site_tail(const Args &a, const Field &fg, uint32
     {   // subgroup (0,1): reads M00 M01 M10 M11
         A q[4];
         quat<A, 0, 1>(M, q);
-        gauge_update<A, G, ALGO>(q, a.param, rng);
+        update(q);
         left_su2<A, 0, 1>(Gx, q);
     }
 
@@ -614,13 +649,12 @@ __device__ __forceinline__ void site_tail(const Args &a, const Field &fg, uint32
     }
 }
 
-// Philox generator of a site (SA, random transformation): key word 0 = global
+// Philox generator of a site (SA): key word 0 = global
 // id of the reference's (mu = 0, up) thread of this site in its V/2/NSB x
 // 8*NSB launch (PhiloxWrapper.hxx:93-110)
 template <typename Args> __device__ __forceinline__ void site_rng(const Args &a, int64_t p, int parity, Philox &rng)
 {
-    const uint32_t tid = (uint32_t)((p / a.nsb) * 8 * a.nsb + p % a.nsb);
-    philox_init(rng, tid, a.seed, a.wf && parity ? a.counter_odd : a.counter);
+    philox_init(rng, rng_tid(p, a.nsb), a.seed, a.wf && parity ? a.counter_odd : a.counter);
 }
 
 // Work mapping 0: a block covers 64 sites with one wave per direction of S
@@ -655,25 +689,20 @@ __device__ __forceinline__ void gsweep_block(const Args &a, int64_t blk, int par
     }
 
     Philox rng;
-    if (ALGO == GF_SA || ALGO == GF_RANDOM) site_rng(a, p, parity, rng);
+    if (ALGO == GF_SA) site_rng(a, p, parity, rng);
 
-    if (ALGO == GF_RANDOM) {
-        // the random transformation does not depend on the links
-        if (wave != 0) return;
-    } else {
-        M3<A> X, Z;
-        direction_terms<A, LF, STREAM>(a, fg, mu, wave, c, par, site, X, Z);
+    M3<A> X, Z;
+    direction_terms<A, LF, STREAM>(a, fg, mu, wave, c, par, site, X, Z);
 #pragma unroll
-        for (int i = 0; i < 3; i++)
+    for (int i = 0; i < 3; i++)
 #pragma unroll
-            for (int j = 0; j < 3; j++) {
-                const int k = 2 * (3 * i + j);
-                lds[((k + 0) * kW + wave) * 64 + lane] = X.e[j][i].x + Z.e[i][j].x;
-                lds[((k + 1) * kW + wave) * 64 + lane] = Z.e[i][j].y - X.e[j][i].y;
-            }
-        __syncthreads();
-        if (wave != 0) return;
-    }
+        for (int j = 0; j < 3; j++) {
+            const int k = 2 * (3 * i + j);
+            lds[((k + 0) * kW + wave) * 64 + lane] = X.e[j][i].x + Z.e[i][j].x;
+            lds[((k + 1) * kW + wave) * 64 + lane] = Z.e[i][j].y - X.e[j][i].y;
+        }
+    __syncthreads();
+    if (wave != 0) return;
 
     // S = sum_mu g(y) U0_mu(x)^dagger + g(z) U0_mu(z), summed in the order of mu
     const auto sum_s = [&](M3<A> &S) {
@@ -693,7 +722,7 @@ __device__ __forceinline__ void gsweep_block(const Args &a, int64_t blk, int par
                 S.e[i][j] = cx(v[0], v[1]);
             }
     };
-    site_tail<A, G, ALGO, THETA, LF>(a, fg, site_off, active, blk, lane, sum_s, Gx, rng, stream_g ? kNt : 0);
+    site_tail<A, G, ALGO, THETA, LF>(a, fg, site_off, active, blk, lane, sum_s, Gx, rng, lds, stream_g ? kNt : 0);
 }
 
 template <typename A, int G, int ALGO, int THETA, int LF, bool STREAM>
@@ -903,8 +932,7 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_pipe(GaugeSweepArgs a)
 
     Philox rng;
     if (ALGO == GF_SA) {  // the key of the site's (mu = 0, up) reference thread; odd sites: counter + 1
-        const uint32_t tid = (uint32_t)((p / a.nsb) * 8 * a.nsb + p % a.nsb);
-        philox_init(rng, tid, a.seed, odd ? a.counter + 1 : a.counter);
+        philox_init(rng, rng_tid(p, a.nsb), a.seed, odd ? a.counter + 1 : a.counter);
     }
     {
         // the direction-mu terms as direction_terms forms them; the neighbours
@@ -952,7 +980,7 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_pipe(GaugeSweepArgs a)
             }
     };
     // even sites: g stored coherently at device scope (read by odd items of this launch)
-    site_tail<A, G, ALGO, 0, LF>(a, fg, site_off, active, blk, lane, sum_s, Gx, rng, odd ? 0 : kSc1);
+    site_tail<A, G, ALGO, 0, LF>(a, fg, site_off, active, blk, lane, sum_s, Gx, rng, lds, odd ? 0 : kSc1);
     if (odd) return;
     // the stores are complete before the flag says so
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -1009,7 +1037,7 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_mag(GaugeSweepArgs a)
     load_g<A, LF>(fg, site_off, Gx);
     third_row(Gx);
     Philox rng;  // wave 0 computes the updates
-    if ((ALGO == GF_SA || ALGO == GF_SR || ALGO == GF_RANDOM) && mu == 0) site_rng(a, p, parity, rng);
+    if (ALGO == GF_SA && mu == 0) site_rng(a, p, parity, rng);
 
     M3<A> up, dn;
     {
@@ -1148,16 +1176,13 @@ template <typename A, int LF> hipError_t launch_mag_lf(int algo, int theta, cons
             if (theta == 1) launch_k_mag<A, GF_OR, 1, LF>(a, s);
             else if (theta == 2) launch_k_mag<A, GF_OR, 2, LF>(a, s);
             else launch_k_mag<A, GF_OR, 0, LF>(a, s);
-        } else if (theta != 0) {
-            return hipErrorInvalidValue;
-        } else if (algo == GF_MICRO) {
-            launch_k_mag<A, GF_MICRO, 0, LF>(a, s);
-        } else if (algo == GF_SA) {
-            launch_k_mag<A, GF_SA, 0, LF>(a, s);
-        } else if (algo == GF_SR) {
-            launch_k_mag<A, GF_SR, 0, LF>(a, s);
-        } else if (algo == GF_RANDOM) {  // MAG's random step keeps q3 = 0 (GaugeFixingSubgroupStep.hxx:566-575)
-            launch_k_mag<A, GF_RANDOM, 0, LF>(a, s);
+            return hipGetLastError();
+        }
+        if constexpr (sizeof(A) == 4) {  // the annealing's updates
+            if (theta != 0) return hipErrorInvalidValue;
+            if (algo == GF_MICRO) launch_k_mag<A, GF_MICRO, 0, LF>(a, s);
+            else if (algo == GF_SA) launch_k_mag<A, GF_SA, 0, LF>(a, s);
+            else return hipErrorInvalidValue;
         } else {
             return hipErrorInvalidValue;
         }
@@ -1171,6 +1196,26 @@ void launch_k(const GaugeSweepArgs &a, hipStream_t s)
     const dim3 grid((unsigned)gsweep_grid(a)), block(64 * gsweep_waves<G>());
     if (gsweep_streams(a)) hipLaunchKernelGGL((k_gsweep<A, G, ALGO, THETA, LF, true>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((k_gsweep<A, G, ALGO, THETA, LF, false>), grid, block, 0, s, a);
+}
+
+// FP32 or 24-bit links: OR of the mixed driver (either arithmetic), SA and
+// microcanonical of the annealing (FP32)
+template <typename A, int G, int LF> hipError_t launch_lf(int algo, int theta, const GaugeSweepArgs &a, hipStream_t s)
+{
+    if (algo == GF_OR) {
+        if (theta == 1) launch_k<A, G, GF_OR, 1, LF>(a, s);
+        else if (theta == 2) launch_k<A, G, GF_OR, 2, LF>(a, s);
+        else launch_k<A, G, GF_OR, 0, LF>(a, s);
+        return hipGetLastError();
+    }
+    if constexpr (sizeof(A) == 4) {
+        if (theta != 0) return hipErrorInvalidValue;
+        if (algo == GF_MICRO) launch_k<A, G, GF_MICRO, 0, LF>(a, s);
+        else if (algo == GF_SA) launch_k<A, G, GF_SA, 0, LF>(a, s);
+        else return hipErrorInvalidValue;
+        return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
 }
 
 template <typename A, int G> hipError_t launch_g(int algo, int theta, const GaugeSweepArgs &a, hipStream_t s)
@@ -1187,36 +1232,7 @@ template <typename A, int G> hipError_t launch_g(int algo, int theta, const Gaug
         return hipErrorInvalidValue;
     }
     if (theta == 3) return hipErrorInvalidValue;
-    if (a.links24) {  // fixed-point links: OR of the mixed driver, SA and microcanonical of the annealing
-        if (algo == GF_OR) {
-            if (theta == 1) launch_k<A, G, GF_OR, 1, 1>(a, s);
-            else if (theta == 2) launch_k<A, G, GF_OR, 2, 1>(a, s);
-            else launch_k<A, G, GF_OR, 0, 1>(a, s);
-        } else if (theta != 0) {
-            return hipErrorInvalidValue;
-        } else if (algo == GF_MICRO) {
-            launch_k<A, G, GF_MICRO, 0, 1>(a, s);
-        } else if (algo == GF_SA) {
-            launch_k<A, G, GF_SA, 0, 1>(a, s);
-        } else {
-            return hipErrorInvalidValue;
-        }
-    } else if (algo == GF_OR) {
-        if (theta == 1) launch_k<A, G, GF_OR, 1, 0>(a, s);
-        else if (theta == 2) launch_k<A, G, GF_OR, 2, 0>(a, s);
-        else launch_k<A, G, GF_OR, 0, 0>(a, s);
-    } else if (theta != 0) {
-        return hipErrorInvalidValue;
-    } else if (algo == GF_MICRO) {
-        launch_k<A, G, GF_MICRO, 0, 0>(a, s);
-    } else if (algo == GF_SA) {
-        launch_k<A, G, GF_SA, 0, 0>(a, s);
-    } else if (algo == GF_RANDOM) {
-        launch_k<A, G, GF_RANDOM, 0, 0>(a, s);
-    } else {
-        return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    return a.links24 ? launch_lf<A, G, 1>(algo, theta, a, s) : launch_lf<A, G, 0>(algo, theta, a, s);
 }
 
 // links (type R, layout SI) -> rows 0,1 in the 24-bit fixed-point form, in

@@ -132,7 +132,7 @@ struct GaugeSweepArgs {
     PipePlan plan;
     FastDiv pipe_tdiv;
 };
-// algo: GF_OR, GF_MICRO, GF_SA or GF_RANDOM; theta (OR only): 0 none,
+// algo: GF_OR, or (FP32 arithmetic) GF_MICRO or GF_SA; theta (OR only): 0 none,
 // 1 pre-update (even kernel), 2 post-update (odd kernel), 3 the read-only
 // theta pass (links64 only, while state->near is set); fp64_arith: compute
 // in FP64 on the FP32 data (required with links64)

@@ -77,6 +77,8 @@ __device__ __forceinline__ double cospi_(double x) { return cospi(x); }
 __device__ __forceinline__ float cospi_(float x) { return cospif(x); }
 __device__ __forceinline__ double sinpi_(double x) { return sinpi(x); }
 __device__ __forceinline__ float sinpi_(float x) { return sinpif(x); }
+__device__ __forceinline__ void sincospi_(double x, double &s, double &c) { sincospi(x, &s, &c); }
+__device__ __forceinline__ void sincospi_(float x, float &s, float &c) { sincospif(x, &s, &c); }
 __device__ __forceinline__ double log_(double x) { return log(x); }
 __device__ __forceinline__ float log_(float x) { return logf(x); }
 
@@ -157,35 +159,155 @@ template <typename R> __device__ __forceinline__ void upd_random(R a[4], Philox 
 // 2.0*rand-1.0 and sqrt(1.0-cos^2) -- with float operands rounded first
 // (r4*r4, cos_theta*cos_theta) and float results; W is that wider type.
 // The fast kernels keep everything in R.
+//
+// One attempt with the uniforms u: delta, and whether it is accepted.
+template <bool E, typename R> __device__ __forceinline__ bool sa_accept(R u1, R u2, R u3, R u4, R p0, R &delta)
+{
+    using W = std::conditional_t<E, double, R>;
+    const R r1 = -log_(u1) * p0;
+    const R r2 = -log_(u2) * p0;
+    R r3 = (R)cospi_((W)2 * (W)u3);
+    r3 = r3 * r3;
+    delta = r2 + r1 * r3;
+    const R r4sq = u4 * u4;
+    return !((W)r4sq > (W)1 - (W)0.5 * (W)delta);
+}
+template <bool E, typename R> __device__ __forceinline__ bool sa_redraw(R u)
+{
+    using W = std::conditional_t<E, double, R>;
+    return (W)u < (W)0.0001;
+}
+
+template <bool E, typename R, typename RAND>
+__device__ __forceinline__ bool sa_attempt(Philox &rng, R p0, R &delta)
+{
+    R u1, u2;
+    do { u1 = (R)philox_rand(rng, RAND(0)); } while (sa_redraw<E>(u1));
+    do { u2 = (R)philox_rand(rng, RAND(0)); } while (sa_redraw<E>(u2));
+    const R u3 = (R)philox_rand(rng, RAND(0));
+    const R u4 = (R)philox_rand(rng, RAND(0));
+    return sa_accept<E>(u1, u2, u3, u4, p0, delta);
+}
+
+// Place of the n-th set bit (n = 0 the lowest) of m; some place where m has no
+// more than n.
+__device__ __forceinline__ int nth_set_bit(uint64_t m, int n)
+{
+    const int lo = __popc((uint32_t)m);
+    const bool high = n >= lo;
+    uint32_t w = high ? (uint32_t)(m >> 32) : (uint32_t)m;
+    int at = high ? 32 : 0;
+    n -= high ? lo : 0;
+#pragma unroll
+    for (int step = 16; step >= 1; step >>= 1) {
+        const int c = __popc(w & ((1u << step) - 1));
+        const bool up = n >= c;
+        w >>= up ? step : 0;
+        at += up ? step : 0;
+        n -= up ? c : 0;
+    }
+    return at;
+}
+
+// The accepted delta of every lane's site; called by a whole wave of 64
+// sites.  A site accepts with a probability that falls with its p0 (below
+// 1e-5 for the smallest sums of links of a hot U1xU1 or MAG lattice), and the
+// wave takes as long as its slowest site.  But a site's attempts are its
+// stream's draws in fours, so they can be made side by side: after
+// kOwnAttempts, once at most half of the lanes still need one, the wave's
+// lanes share out the sites left, each group of lanes making one site's next
+// attempts, and the site takes the first that is accepted.  Its stream goes
+// on after that attempt, so delta and every later draw are those of the
+// attempts made one after another.  (An attempt whose first or second draw is
+// drawn again takes more than four draws: the site makes that one itself.)
+// U1xU1 heatbath half-sweep at T = 2.4, FP64: 8^4 8.0 ms -> 0.10 ms, 32^4 93
+// -> 1.1 ms; FP32 32^4 107 -> 1.4 ms; one temperature of the annealing on
+// 24-bit links, 16^4: U1xU1 15 -> 0.42 ms, MAG 0.375 -> 0.344 ms.  Where
+// nearly every first attempt is accepted (Landau at T = 0.3) it changes
+// nothing.
+constexpr int kOwnAttempts = 3;  // 2 to 4 measure the same
+template <bool E, typename R, typename RAND> __device__ __forceinline__ R sa_delta(Philox &rng, R p0)
+{
+    const int lane = threadIdx.x & 63;
+    R delta;
+    bool done = sa_attempt<E, R, RAND>(rng, p0, delta);
+    uint64_t left = __ballot(!done);
+    for (int own = 1; left && (own < kOwnAttempts || __popcll(left) > 32); own++) {
+        if (!done) done = sa_attempt<E, R, RAND>(rng, p0, delta);
+        left = __ballot(!done);
+    }
+    if (!left) return delta;
+    uint32_t pos = philox_pos<RAND>(rng);  // draws taken by the site's attempts so far
+    while (left) {
+        const int n = __popcll(left);
+        const int lg = n == 1 ? 6 : __builtin_clz(n - 1) - 26;  // 2^lg lanes to a site: 64 / n rounded down
+        const int rank = __popcll(left & ((uint64_t(1) << lane) - 1));  // of an unfinished lane
+        const int group = lane >> lg, j = lane & ((1 << lg) - 1);
+        const int src = nth_set_bit(left, group);  // the lane whose site the group works on
+        const R p0s = __shfl(p0, src, 64);
+        R u[4];
+        {
+            RAND v[4];
+            philox_at((uint32_t)__shfl((int)rng.k0, src, 64), rng.k1, rng.c1,
+                      (uint32_t)__shfl((int)pos, src, 64) + 4 * (uint32_t)j, v);
+#pragma unroll
+            for (int k = 0; k < 4; k++) u[k] = (R)v[k];
+        }
+        R d;
+        const bool acc = sa_accept<E>(u[0], u[1], u[2], u[3], p0s, d);
+        const bool again = sa_redraw<E>(u[0]) || sa_redraw<E>(u[1]);
+        const uint64_t good = __ballot(group < n && acc && !again), redo = __ballot(group < n && again);
+        int first = 64;  // the lane whose attempt the site takes
+        bool own = false;
+        if (!done) {
+            const uint64_t mine = lg == 6 ? ~uint64_t(0) : ((uint64_t(1) << (1 << lg)) - 1) << (rank << lg);
+            const int a = (good & mine) ? __ffsll((unsigned long long)(good & mine)) - 1 : 64;
+            const int b = (redo & mine) ? __ffsll((unsigned long long)(redo & mine)) - 1 : 64;
+            if (a < b) {
+                first = a;
+                pos += 4 * (uint32_t)(a - (rank << lg) + 1);
+            } else {
+                own = b < 64;
+                pos += 4 * (uint32_t)(own ? b - (rank << lg) : 1 << lg);
+            }
+        }
+        const R taken = __shfl(d, first & 63, 64);
+        if (first < 64) {
+            delta = taken;
+            done = true;
+            philox_seek<RAND>(rng, pos);
+        } else if (own) {
+            philox_seek<RAND>(rng, pos);
+            done = sa_attempt<E, R, RAND>(rng, p0, delta);
+            pos = philox_pos<RAND>(rng);
+        }
+        left = __ballot(!done);
+    }
+    return delta;
+}
+
 template <bool E, typename R, typename RAND = R>
 __device__ __forceinline__ void upd_sa(R a[4], float temperature, Philox &rng)
 {
     using W = std::conditional_t<E, double, R>;
     R e0 = a[0], e1 = -a[1], e2 = -a[2], e3 = -a[3];
     const R dk = inv_sqrt<E>(e0 * e0 + e1 * e1 + e2 * e2 + e3 * e3);
-    const R p0 = dk * (R)temperature;
-    R delta;
-    for (;;) {
-        R r1, r2;
-        do { r1 = (R)philox_rand(rng, RAND(0)); } while ((W)r1 < (W)0.0001);
-        r1 = -log_(r1) * p0;
-        do { r2 = (R)philox_rand(rng, RAND(0)); } while ((W)r2 < (W)0.0001);
-        r2 = -log_(r2) * p0;
-        R r3 = (R)cospi_((W)2 * (W)(R)philox_rand(rng, RAND(0)));
-        r3 = r3 * r3;
-        delta = r2 + r1 * r3;
-        const R r4 = (R)philox_rand(rng, RAND(0));
-        const R r4sq = r4 * r4;
-        if (!((W)r4sq > (W)1 - (W)0.5 * (W)delta)) break;
-    }
+    const R delta = sa_delta<E, R, RAND>(rng, dk * (R)temperature);
     const R b0 = (R)((W)1 - (W)delta);
     const R cos_theta = (R)((W)2 * (W)(R)philox_rand(rng, RAND(0)) - (W)1);
     const R cos_sq = cos_theta * cos_theta;
     const R sin_theta = (R)sqrt_((W)1 - (W)cos_sq);
     const R sin_alpha = sqrt_((R)1 - b0 * b0);
     const R phi = (R)((W)2 * (W)(R)philox_rand(rng, RAND(0)));
-    const R b1 = sin_alpha * sin_theta * cospi_(phi);
-    const R b2 = sin_alpha * sin_theta * sinpi_(phi);
+    R sin_phi, cos_phi;
+    if constexpr (E) {  // sincospi's values are sinpi's and cospi's, from one reduction
+        sincospi_(phi, sin_phi, cos_phi);
+    } else {  // (with contraction the shared reduction would round differently)
+        cos_phi = cospi_(phi);
+        sin_phi = sinpi_(phi);
+    }
+    const R b1 = sin_alpha * sin_theta * cos_phi;
+    const R b2 = sin_alpha * sin_theta * sin_phi;
     const R b3 = sin_alpha * cos_theta;
     e0 *= dk;
     e1 *= dk;
@@ -443,6 +565,7 @@ template <typename R, int G, int A, int S, bool EXACT, int THETA, bool GACC, boo
 __global__ __launch_bounds__(kBlock) void k_sweep(SweepArgs<R> a)
 {
     static_assert(!EXACT || THETA == 0, "the reference-order kernels carry no fused check");
+    static_assert(A % kDpUpdate == GF_OR || A % kDpUpdate == GF_MICRO, "k_sweep_rng makes the updates with random numbers");
     constexpr int kTerms = EXACT ? 8 : 4;   // exchanged per site: links, or directions
     constexpr int kQ = kTerms * 4 * 64;     // one exchange buffer: [term][comp 4][lane 64]
     constexpr int kT = kThetaVals * 4 * 64;
@@ -499,13 +622,7 @@ __global__ __launch_bounds__(kBlock) void k_sweep(SweepArgs<R> a)
         }
     }
 
-    Philox rng;
-    constexpr int AB = A % kDpUpdate;  // the update rule without its precision
-    if (AB == GF_SA || AB == GF_SR || AB == GF_RANDOM) {
-        // key word 0 = global thread id of the reference's (mu=0, down=0) thread
-        const uint32_t tid = (uint32_t)((p / a.nsb) * 8 * a.nsb + p % a.nsb);
-        philox_init(rng, tid, a.seed, a.counter);
-    }
+    Philox rng;  // (these updates draw no random numbers)
 
     // fused check: each wave writes its direction's terms to the check's own
     // LDS area, and wave 0 adds them at the end of the kernel, after a barrier
