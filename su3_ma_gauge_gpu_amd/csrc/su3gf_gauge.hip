@@ -1012,9 +1012,8 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_mag(GaugeSweepArgs a)
     __shared__ A lds[2 * kX + 4 * 64 + (THETA ? kThetaVals * 4 * 64 : 0)];
     A *const qlds = lds + 2 * kX;  // the update: [q0..q3][lane 64]
     A *const tlds = qlds + 4 * 64;
-    static_assert(LF != 2 || sizeof(A) == 8, "FP64 storage takes FP64 arithmetic");
+    static_assert(LF != 2 && THETA != 3, "FP32 or 24-bit links; k_gsweep_mag64 sweeps the FP64 ones");
     if (a.state && a.state->done) return;  // converged: uniform early exit
-    if (THETA == 3 && !a.state->near) return;
     const int mu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     int parity = a.parity;
@@ -1064,17 +1063,7 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_mag(GaugeSweepArgs a)
             if (active) theta_site<GF_MAG>(s3, th, gf);
         }
     };
-    if (THETA == 1 || THETA == 3) theta_pass();
-    if constexpr (THETA == 3) {  // read-only pass: theta only
-        if (mu != 0) return;
-        th = wave64_sum(th);
-        gf = wave64_sum(gf);
-        if (lane == 0) {
-            a.partial[2 * blk] = th;
-            a.partial[2 * blk + 1] = gf;
-        }
-        return;
-    }
+    if (THETA == 1) theta_pass();
 
     int buf = 0;
     auto subgroup = [&](auto I_, auto J_) {
@@ -1139,6 +1128,248 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_mag(GaugeSweepArgs a)
     }
 }
 
+// MAG in FP64 on the FP64 links (the FP64 phase), on sums over the links as for
+// the other gauges.  With W = U_up for a site's up links and W = U_down^dagger
+// for its down links, every update is W <- G W, and the quadratic forms that
+// MAG needs are entries of the Hermitian matrices P_c = sum of the outer
+// products w w^dagger of column c of W over the eight links: for the subgroup
+// (i, j) D = (P_i - P_j)_ii - (P_i - P_j)_jj and c = (P_i - P_j)_ij, theta_x's
+// X_ij is that c, and the functional's sum of |U_jj|^2 is the sum of (P_j)_jj.
+// W is unitary, so P_2 = 8 - P_0 - P_1, and only columns 0 and 1 are formed.
+// Wave mu forms its two links' columns without g(x) -- of U0_mu(x) g(y)^dagger,
+// and rows 0, 1 of g(z) U0_mu(z), conjugated -- and their outer products, 18
+// reals that go through LDS; wave 0 adds the four, rotates the sums by g(x) and
+// makes the three updates on them (P_c <- G P_c G^dagger) and on g(x).  The
+// four waves thus stop after their products (about 370 of the 1220 to 1640
+// VALU instructions per wave of the sweep on the links themselves, as
+// k_gsweep_mag makes it, where every wave turns its links by g(x) and by the
+// three updates), with one barrier instead of six: 24^4 42.6 -> 31.7 us per
+// checked launch, 32^4 130 -> 94, 48^4 687 -> 566, which is the Landau sweep's
+// time (31, 92, 559): the bytes bound it now.
+template <typename A> struct Outer {
+    A d[3];       // the diagonal
+    Cx<A> o[3];   // (0,1), (0,2), (1,2)
+};
+// += w w^dagger
+template <typename A> __device__ __forceinline__ void add_outer(Outer<A> &P, const Cx<A> w[3])
+{
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        P.d[i] = fma_(w[i].x, w[i].x, P.d[i]);
+        P.d[i] = fma_(w[i].y, w[i].y, P.d[i]);
+    }
+    cmacc(P.o[0], w[0], w[1]);
+    cmacc(P.o[1], w[0], w[2]);
+    cmacc(P.o[2], w[1], w[2]);
+}
+// P <- g P g^dagger
+template <typename A> __device__ __forceinline__ void turn(Outer<A> &P, const M3<A> &g)
+{
+    M3<A> T;  // g P
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        T.e[i][0] = g.e[i][0] * P.d[0];
+        cmacc(T.e[i][0], g.e[i][1], P.o[0]);
+        cmacc(T.e[i][0], g.e[i][2], P.o[1]);
+        T.e[i][1] = g.e[i][1] * P.d[1];
+        cmac(T.e[i][1], g.e[i][0], P.o[0]);
+        cmacc(T.e[i][1], g.e[i][2], P.o[2]);
+        T.e[i][2] = g.e[i][2] * P.d[2];
+        cmac(T.e[i][2], g.e[i][0], P.o[1]);
+        cmac(T.e[i][2], g.e[i][1], P.o[2]);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        A d = 0;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            d = fma_(T.e[i][k].x, g.e[i][k].x, d);
+            d = fma_(T.e[i][k].y, g.e[i][k].y, d);
+        }
+        P.d[i] = d;
+    }
+#pragma unroll
+    for (int m = 0; m < 3; m++) {
+        const int i = m == 2 ? 1 : 0, j = m == 0 ? 1 : 2;
+        Cx<A> s = czero<A>();
+#pragma unroll
+        for (int k = 0; k < 3; k++) cmacc(s, T.e[i][k], g.e[j][k]);
+        P.o[m] = s;
+    }
+}
+// P <- G P G^dagger for the SU(2) element q of subgroup (I, J), whose q3 is 0:
+// G = [[q0, s], [-conj(s), q0]] with s = q2 + i q1
+template <typename A, int I, int J> __device__ __forceinline__ void turn_su2(Outer<A> &P, const A q[4])
+{
+    const Cx<A> s = cx(q[2], q[1]);
+    const A c2 = q[0] * q[0], s2 = fma_(s.x, s.x, s.y * s.y);
+    constexpr int IJ = I + J - 1;  // of the off-diagonal entry (I, J)
+    const A a = P.d[I], d = P.d[J];
+    const Cx<A> b = P.o[IJ];
+    const A cross = (A)2 * q[0] * fma_(s.x, b.x, s.y * b.y);  // 2 q0 Re(s conj(b))
+    P.d[I] = fma_(c2, a, fma_(s2, d, cross));
+    P.d[J] = fma_(s2, a, fma_(c2, d, -cross));
+    const Cx<A> ss = s * s;  // b' = q0^2 b - s^2 conj(b) + q0 s (d - a)
+    Cx<A> n = s * (q[0] * (d - a));
+    n.x = fma_(c2, b.x, n.x);
+    n.y = fma_(c2, b.y, n.y);
+    cmacc(n, cx(-ss.x, -ss.y), b);
+    P.o[IJ] = n;
+    // the entries with the third index K: (I, K) and (J, K)
+    constexpr int K = 3 - I - J;
+    const auto entry = [&](int r) -> Cx<A> { return r < K ? P.o[r + K - 1] : conj(P.o[r + K - 1]); };
+    const Cx<A> u = entry(I), v = entry(J);
+    Cx<A> nu = u * q[0], nv = v * q[0];
+    cmac(nu, s, v);
+    cmac(nv, cx(-s.x, s.y), u);
+    P.o[I + K - 1] = I < K ? nu : conj(nu);
+    P.o[J + K - 1] = J < K ? nv : conj(nv);
+}
+
+template <int THETA, bool STREAM>
+__global__ __launch_bounds__(kGBlock) void k_gsweep_mag64(GaugeSweepArgs a)
+{
+    using A = double;
+    __shared__ A lds[18 * 4 * 64];
+    if (a.state && a.state->done) return;  // converged: uniform early exit
+    if (THETA == 3 && !a.state->near) return;
+    const int mu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    int parity = a.parity;
+    int64_t blk;
+    if (a.wf) {
+        if (!wave_block(a, blk, parity)) return;
+    } else {
+        blk = ordered_block(a.order, blockIdx.x);
+        if (blk < 0) return;
+    }
+    bool active;
+    const int64_t p = block_site(a.geo, blk, lane, active);
+    const int64_t site = (active ? p : 0) + (parity ? a.geo.Vh : 0);
+    int c[4], par;
+    site_coords(a.geo, site, c, par);
+    const uint32_t site_off = site_boff<2>(site);
+    const Field fg = g_field<2>(a);
+    bool stream_g = false, kx = true, kz = true;
+    const int64_t z = backward(a.geo, c, par, mu);
+    if constexpr (STREAM) {  // as gsweep_block and direction_terms
+        stream_g = a.stream_g;
+        kx = kept_link(a.keep, a.geo.Vh, par ? site - a.geo.Vh : site, mu);
+        kz = kept_link(a.keep, a.geo.Vh, par ? z : z - a.geo.Vh, mu);
+    }
+    M3<A> Gx;
+    if (mu == 0) {
+        if (stream_g) load_g<A, 2, kNt>(fg, site_off, Gx);
+        else load_g<A, 2>(fg, site_off, Gx);
+    }
+    {
+        Outer<A> P[2] = {};
+        M3<A> T, W;
+        const uint32_t y_off = site_boff<2>(forward(a.geo, c, par, mu)), z_off = site_boff<2>(z);
+        const Field fu = links_field<2>(a.U0, a.geo.V, mu);
+        load_links<A, 2, STREAM>(fu, site_off, W, kx);
+        load_g<A, 2>(fg, y_off, T);
+        third_row(W);
+#pragma unroll
+        for (int k = 0; k < 2; k++) {  // column k of U0_mu(x) g(y)^dagger
+            Cx<A> w[3];
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                w[i] = czero<A>();
+#pragma unroll
+                for (int j = 0; j < 3; j++) cmacc(w[i], W.e[i][j], T.e[k][j]);
+            }
+            add_outer(P[k], w);
+        }
+        load_g<A, 2>(fg, z_off, T);
+        load_links<A, 2, STREAM>(fu, z_off, W, kz);
+        third_row(W);
+#pragma unroll
+        for (int k = 0; k < 2; k++) {  // row k of g(z) U0_mu(z), conjugated
+            Cx<A> w[3];
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                w[i] = czero<A>();
+#pragma unroll
+                for (int j = 0; j < 3; j++) cmac(w[i], T.e[k][j], W.e[j][i]);
+                w[i] = conj(w[i]);
+            }
+            add_outer(P[k], w);
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                A *const b = lds + (9 * k + 3 * i) * 256 + mu * 64 + lane;
+                b[0] = P[k].d[i];
+                b[256] = P[k].o[i].x;
+                b[512] = P[k].o[i].y;
+            }
+    }
+    __syncthreads();
+    if (mu != 0) return;
+    third_row(Gx);
+    Outer<A> P[2];
+    const auto sum = [&](int v) {  // value v of the four directions, in the order of mu
+        const A *const b = lds + v * 256 + lane;
+        return ((b[0] + b[64]) + b[128]) + b[192];
+    };
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            P[k].d[i] = sum(9 * k + 3 * i);
+            P[k].o[i] = cx(sum(9 * k + 3 * i + 1), sum(9 * k + 3 * i + 2));
+        }
+        turn(P[k], Gx);
+    }
+    // the subgroups' c = X_ij, and D (P_2 = 8 - P_0 - P_1)
+    const auto x01 = [&] { return P[0].o[0] - P[1].o[0]; };
+    const auto x02 = [&] { return P[0].o[1] * (A)2 + P[1].o[1]; };
+    const auto x12 = [&] { return P[1].o[2] * (A)2 + P[0].o[2]; };
+    const auto theta = [&]() {
+        const Cx<A> x[3] = {x01(), x02(), x12()};
+        double s[kThetaVals];
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            s[2 * k] = x[k].x;
+            s[2 * k + 1] = x[k].y;
+        }
+        s[9] = (P[0].d[0] + P[1].d[1]) + ((A)8 - (P[0].d[2] + P[1].d[2]));
+        double th = 0, gf = 0;
+        if (active) theta_site<GF_MAG>(s, th, gf);
+        th = wave64_sum(th);
+        gf = wave64_sum(gf);
+        if (lane == 0) {
+            a.partial[2 * blk] = th;
+            a.partial[2 * blk + 1] = gf;
+        }
+    };
+    if (THETA == 1 || THETA == 3) theta();  // the state before the update
+    if constexpr (THETA != 3) {
+        Philox rng;  // overrelaxation draws no random numbers
+        A q[4];
+        const auto update = [&](A D, Cx<A> x) { finish_update<A, GF_MAG, GF_OR, false>(D, x.y, x.x, (A)0, q, a.param, rng); };
+        update((A)2 * (P[0].d[0] - P[0].d[2]) + (P[1].d[0] - P[1].d[2]), x02());
+        turn_su2<A, 0, 2>(P[0], q);
+        turn_su2<A, 0, 2>(P[1], q);
+        left_su2<A, 0, 2>(Gx, q);
+        update((A)2 * (P[1].d[1] - P[1].d[2]) + (P[0].d[1] - P[0].d[2]), x12());
+        turn_su2<A, 1, 2>(P[0], q);
+        turn_su2<A, 1, 2>(P[1], q);
+        left_su2<A, 1, 2>(Gx, q);
+        update((P[0].d[0] - P[0].d[1]) - (P[1].d[0] - P[1].d[1]), x01());
+        left_su2<A, 0, 1>(Gx, q);
+        if (THETA == 2) {
+            turn_su2<A, 0, 1>(P[0], q);
+            turn_su2<A, 0, 1>(P[1], q);
+            theta();
+        }
+        project_rows01(Gx);
+        if (active) store_g<A, 2>(fg, site_off, Gx, stream_g ? kNt : 0);
+    }
+}
+
 // blocks of a launch: one per logical block, or a wavefront launch's even and odd grids
 inline int64_t gsweep_grid(const GaugeSweepArgs &a)
 {
@@ -1157,37 +1388,41 @@ template <typename A, int ALGO, int THETA, int LF> void launch_k_mag(const Gauge
     else hipLaunchKernelGGL((k_gsweep_mag<A, ALGO, THETA, LF, false>), grid, block, 0, s, a);
 }
 
+// FP64 links and g: the FP64 phase, OR with the check, or the read-only theta pass
+template <int THETA> void launch_k_mag64(const GaugeSweepArgs &a, hipStream_t s)
+{
+    const dim3 grid((unsigned)gsweep_grid(a)), block(kGBlock);
+    if (gsweep_streams(a)) hipLaunchKernelGGL((k_gsweep_mag64<THETA, true>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((k_gsweep_mag64<THETA, false>), grid, block, 0, s, a);
+}
+
+hipError_t launch_mag64(int algo, int theta, const GaugeSweepArgs &a, hipStream_t s)
+{
+    if (algo != GF_OR) return hipErrorInvalidValue;
+    if (theta == 1) launch_k_mag64<1>(a, s);
+    else if (theta == 2) launch_k_mag64<2>(a, s);
+    else if (theta == 3) launch_k_mag64<3>(a, s);
+    else launch_k_mag64<0>(a, s);
+    return hipGetLastError();
+}
+
 template <typename A, int LF> hipError_t launch_mag_lf(int algo, int theta, const GaugeSweepArgs &a, hipStream_t s)
 {
-    if constexpr (LF == 2) {  // the FP64 phase: OR with the check, or the read-only theta pass
-        if constexpr (sizeof(A) != 8) {
-            return hipErrorInvalidValue;
-        } else {
-            if (algo != GF_OR) return hipErrorInvalidValue;
-            if (theta == 1) launch_k_mag<A, GF_OR, 1, 2>(a, s);
-            else if (theta == 2) launch_k_mag<A, GF_OR, 2, 2>(a, s);
-            else if (theta == 3) launch_k_mag<A, GF_OR, 3, 2>(a, s);
-            else launch_k_mag<A, GF_OR, 0, 2>(a, s);
-            return hipGetLastError();
-        }
-    } else {
-        if (theta == 3) return hipErrorInvalidValue;
-        if (algo == GF_OR) {
-            if (theta == 1) launch_k_mag<A, GF_OR, 1, LF>(a, s);
-            else if (theta == 2) launch_k_mag<A, GF_OR, 2, LF>(a, s);
-            else launch_k_mag<A, GF_OR, 0, LF>(a, s);
-            return hipGetLastError();
-        }
-        if constexpr (sizeof(A) == 4) {  // the annealing's updates
-            if (theta != 0) return hipErrorInvalidValue;
-            if (algo == GF_MICRO) launch_k_mag<A, GF_MICRO, 0, LF>(a, s);
-            else if (algo == GF_SA) launch_k_mag<A, GF_SA, 0, LF>(a, s);
-            else return hipErrorInvalidValue;
-        } else {
-            return hipErrorInvalidValue;
-        }
+    if (theta == 3) return hipErrorInvalidValue;
+    if (algo == GF_OR) {
+        if (theta == 1) launch_k_mag<A, GF_OR, 1, LF>(a, s);
+        else if (theta == 2) launch_k_mag<A, GF_OR, 2, LF>(a, s);
+        else launch_k_mag<A, GF_OR, 0, LF>(a, s);
         return hipGetLastError();
     }
+    if constexpr (sizeof(A) == 4) {  // the annealing's updates
+        if (theta != 0) return hipErrorInvalidValue;
+        if (algo == GF_MICRO) launch_k_mag<A, GF_MICRO, 0, LF>(a, s);
+        else if (algo == GF_SA) launch_k_mag<A, GF_SA, 0, LF>(a, s);
+        else return hipErrorInvalidValue;
+        return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
 }
 
 template <typename A, int G, int ALGO, int THETA, int LF>
@@ -1269,7 +1504,7 @@ template <typename R, int SI> __global__ __launch_bounds__(256) void k_pack24(co
 template <typename A> hipError_t launch_a(int gauge, int algo, int theta, const GaugeSweepArgs &a, hipStream_t s)
 {
     if (gauge == GF_MAG) {
-        if (a.links64) return launch_mag_lf<A, 2>(algo, theta, a, s);
+        if (a.links64) return sizeof(A) == 8 ? launch_mag64(algo, theta, a, s) : hipErrorInvalidValue;
         return a.links24 ? launch_mag_lf<A, 1>(algo, theta, a, s) : launch_mag_lf<A, 0>(algo, theta, a, s);
     }
     if (gauge == GF_LANDAU) return launch_g<A, GF_LANDAU>(algo, theta, a, s);
