@@ -225,9 +225,9 @@ struct gf_stats {
     int crit;
     int64_t V;
     int64_t nblocks;
-    double *partial;   // device, 2 * nblocks
-    double *out;       // device, 2
-    double *host;      // pinned host, 2
+    double *partial;       // device, 2 * nblocks
+    uint32_t *finished;    // device, 1: the quality kernel's count of finished blocks, 0 between calls
+    QualityResult *host;   // pinned host, written by the kernel
 };
 
 extern "C" {
@@ -484,11 +484,12 @@ gf_status gf_stats_create(const int dims[4], int gauge, int crit, gf_stats **out
     st->V = V;
     st->nblocks = exact::quality_blocks(V);
     hipError_t e = hipMalloc((void **)&st->partial, sizeof(double) * 2 * st->nblocks);
-    if (e == hipSuccess) e = hipMalloc((void **)&st->out, sizeof(double) * 2);
-    if (e == hipSuccess) e = hipHostMalloc((void **)&st->host, sizeof(double) * 2, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipMalloc((void **)&st->finished, sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMemset(st->finished, 0, sizeof(uint32_t));
+    if (e == hipSuccess) e = hipHostMalloc((void **)&st->host, sizeof(QualityResult), hipHostMallocCoherent);
     if (e != hipSuccess) {
         if (st->partial) (void)hipFree(st->partial);
-        if (st->out) (void)hipFree(st->out);
+        if (st->finished) (void)hipFree(st->finished);
         delete st;
         return hip_fail(e, "stats scratch allocation");
     }
@@ -499,7 +500,7 @@ gf_status gf_stats_create(const int dims[4], int gauge, int crit, gf_stats **out
 gf_status gf_stats_destroy(gf_stats *st)
 {
     if (!st) return GF_OK;
-    hipError_t e1 = hipFree(st->partial), e2 = hipFree(st->out), e3 = hipHostFree(st->host);
+    hipError_t e1 = hipFree(st->partial), e2 = hipFree(st->finished), e3 = hipHostFree(st->host);
     delete st;
     if (e1 != hipSuccess) return hip_fail(e1, "hipFree");
     if (e2 != hipSuccess) return hip_fail(e2, "hipFree");
@@ -513,7 +514,7 @@ namespace {
 int quality_tpass(const gf_lattice *lat, int gauge, const void *U, hipStream_t s);
 
 hipError_t quality_kernel(const gf_lattice *lat, int gauge, const void *U, double *dGff, double *dA,
-                          double *partial, int crit_max, int tpass, hipStream_t s)
+                          double *partial, gf_stats *st, int crit_max, int tpass, hipStream_t s)
 {
     int64_t V = 1;
     for (int d = 0; d < 4; d++) V *= lat->dims[d];
@@ -522,23 +523,26 @@ hipError_t quality_kernel(const gf_lattice *lat, int gauge, const void *U, doubl
     if (lat->dtype == GF_F64) {
         QualityArgs<double> a{};
         a.U = (const double *)U; a.g = g; a.dGff = dGff; a.dA = dA; a.partial = partial; a.crit_max = crit_max;
+        if (st) { a.out = st->host; a.finished = st->finished; }
         a.tpass = tpass;
         return exact::launch_quality<double>(lat->layout, gauge, a, s);
     }
     QualityArgs<float> a{};
     a.U = (const float *)U; a.g = g; a.dGff = dGff; a.dA = dA; a.partial = partial; a.crit_max = crit_max;
+    if (st) { a.out = st->host; a.finished = st->finished; }
     a.tpass = tpass;
     return exact::launch_quality<float>(lat->layout, gauge, a, s);
 }
 }  // namespace
 
 static gf_status quality_launch(const gf_lattice *lat, int gauge, const void *U, double *dGff, double *dA,
-                                double *partial, int crit_max, hipStream_t s)
+                                double *partial, gf_stats *st, int crit_max, hipStream_t s)
 {
     int64_t V;
     GF_TRY(check_lattice(lat, &V));
     if (!U) return fail(GF_ERR_BAD_ARG, "U is null");
-    const hipError_t e = quality_kernel(lat, gauge, U, dGff, dA, partial, crit_max, quality_tpass(lat, gauge, U, s), s);
+    const hipError_t e = quality_kernel(lat, gauge, U, dGff, dA, partial, st, crit_max,
+                                        quality_tpass(lat, gauge, U, s), s);
     if (e != hipSuccess) return hip_fail(e, "quality kernel launch");
     return GF_OK;
 }
@@ -551,17 +555,14 @@ gf_status gf_stats_quality(gf_stats *st, const gf_lattice *lat, const void *U, d
     for (int i = 0; i < 4; i++)
         if (lat->dims[i] != st->dims[i]) return fail(GF_ERR_BAD_SHAPE, "lattice shape differs from the stats shape");
     const int crit_max = st->crit == GF_CRIT_MAX;
-    GF_TRY(quality_launch(lat, st->gauge, U, nullptr, nullptr, st->partial, crit_max, S(stream)));
-    hipError_t e = launch_reduce_final(st->partial, st->nblocks, crit_max, st->out, S(stream));
-    if (e != hipSuccess) return hip_fail(e, "reduction kernel launch");
-    HIP_TRY(hipMemcpyAsync(st->host, st->out, 2 * sizeof(double), hipMemcpyDeviceToHost, S(stream)));
+    GF_TRY(quality_launch(lat, st->gauge, U, nullptr, nullptr, st->partial, st, crit_max, S(stream)));
     HIP_TRY(hipStreamSynchronize(S(stream)));
     // GaugeFixingStats.hxx:203-206 with the per-gauge prefactors
     const double Nc = 3.0, Ndim = 4.0;
     const double pg = st->gauge == GF_COULOMB ? 1. / (Nc * (Ndim - 1)) : 1. / (Nc * Ndim);
-    double a = st->host[0] * (1. / Nc);
+    double a = st->host->theta * (1. / Nc);
     if (st->crit == GF_CRIT_AVERAGE) a = a / (double)st->V;
-    if (gff) *gff = st->host[1] * pg / (double)st->V;
+    if (gff) *gff = st->host->gff * pg / (double)st->V;
     if (theta) *theta = a;
     return GF_OK;
 }
@@ -570,7 +571,7 @@ gf_status gf_quality_per_site(const gf_lattice *lat, int gauge, const void *U, d
 {
     if (!dGff || !dA) return fail(GF_ERR_BAD_ARG, "per-site output is null");
     if (gauge < GF_LANDAU || gauge > GF_U1XU1) return fail(GF_ERR_BAD_ARG, "unknown gauge %d", gauge);
-    return quality_launch(lat, gauge, U, dGff, dA, nullptr, 0, S(stream));
+    return quality_launch(lat, gauge, U, dGff, dA, nullptr, nullptr, 0, S(stream));
 }
 
 // ------------------------------------------------------------ drivers
@@ -872,10 +873,10 @@ int quality_tpass(const gf_lattice *lat, int gauge, const void *U, hipStream_t s
     EventPair ev;
     if (!spans.empty() && hipEventCreate(&ev.a) == hipSuccess && hipEventCreate(&ev.b) == hipSuccess) {
         auto time = [&](int P) -> float {
-            if (quality_kernel(lat, gauge, U, nullptr, nullptr, nullptr, 0, P, s) != hipSuccess) return -1.f;
+            if (quality_kernel(lat, gauge, U, nullptr, nullptr, nullptr, nullptr, 0, P, s) != hipSuccess) return -1.f;
             if (hipEventRecord(ev.a, s) != hipSuccess) return -1.f;
             for (int k = 0; k < 3; k++)
-                if (quality_kernel(lat, gauge, U, nullptr, nullptr, nullptr, 0, P, s) != hipSuccess) return -1.f;
+                if (quality_kernel(lat, gauge, U, nullptr, nullptr, nullptr, nullptr, 0, P, s) != hipSuccess) return -1.f;
             float ms = 0;
             if (hipEventRecord(ev.b, s) != hipSuccess || hipEventSynchronize(ev.b) != hipSuccess ||
                 hipEventElapsedTime(&ms, ev.a, ev.b) != hipSuccess)
@@ -1688,7 +1689,7 @@ gf_status gf_time_sweeps(const gf_lattice *lat, void *U, int gauge, int nsweeps,
         const int warm = std::max(2, nsweeps / 2);
         for (int k = 0; k < warm + nsweeps; k++) {
             if (k == warm) HIP_TRY(hipEventRecord(ev.a, s));
-            GF_TRY(quality_launch(lat, gauge, U, nullptr, nullptr, part.as<double>(), 0, s));
+            GF_TRY(quality_launch(lat, gauge, U, nullptr, nullptr, part.as<double>(), nullptr, 0, s));
         }
         HIP_TRY(hipEventRecord(ev.b, s));
         float ms = 0;

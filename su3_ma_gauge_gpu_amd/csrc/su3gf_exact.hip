@@ -334,7 +334,7 @@ __device__ __forceinline__ void load_site_link(const QualityArgs<R> &a, int64_t 
     reconstruct_e<true>(u);
 }
 
-template <typename R, int G, int S>
+template <typename R, int G, int S, bool SMALL>
 __device__ __forceinline__ void quality_site(const QualityArgs<R> &a, int64_t site, double &dA, double &dGff)
 {
     int c[4], par;
@@ -342,7 +342,7 @@ __device__ __forceinline__ void quality_site(const QualityArgs<R> &a, int64_t si
     if (G == GF_MAG) {
         double gff = 0.0;
         double Xx[3] = {0, 0, 0}, Xy[3] = {0, 0, 0};
-#pragma unroll 1
+#pragma unroll(SMALL ? 4 : 1)
         for (int mu = 0; mu < 4; mu++) {
             M3<R> up, dw;
             load_site_link<R, S>(a, site, mu, up);
@@ -382,7 +382,7 @@ __device__ __forceinline__ void quality_site(const QualityArgs<R> &a, int64_t si
     double result = 0;
     // one direction's two links at a time (140 VGPRs in FP64, 3 waves per
     // SIMD); unrolled, all eight links' loads are hoisted (256 VGPRs, 1 wave)
-#pragma unroll 1
+#pragma unroll(SMALL ? 4 : 1)
     for (int mu = mu0; mu < 4; mu++) {
         M3<R> t;
         load_site_link<R, S>(a, site, mu, t);
@@ -428,7 +428,73 @@ __device__ __forceinline__ void quality_site(const QualityArgs<R> &a, int64_t si
 
 constexpr int kQualitySites = 128;  // sites of each parity per block
 
-template <typename R, int G, int S>
+// (theta, gff) of the lattice from its n blocks' partials in a fixed order: sum
+// k (k = 0..1023) takes partials k, k + 1024, ... in order, then a fixed tree.
+// NT threads make them, a thread 1024 / NT of the sums.  They go to host
+// memory that the device maps.  COHERENT: partials of blocks of the same
+// launch, on any XCD.
+template <int NT, bool COHERENT>
+__device__ __forceinline__ void reduce_partials(const double *partial, int64_t n, int crit_max, QualityResult *out)
+{
+    __shared__ double st[NT], sg[NT];
+    constexpr int kV = 1024 / NT;
+    const int t = threadIdx.x;
+    const auto read = [&](int64_t k) {
+        if (!COHERENT) return partial[k];
+        return __longlong_as_double((int64_t)__hip_atomic_load((const uint64_t *)partial + k, __ATOMIC_RELAXED,
+                                                               __HIP_MEMORY_SCOPE_AGENT));
+    };
+    const auto join = [&](double x, double y) { return crit_max ? fmax(x, y) : x + y; };
+    double T[kV], F[kV];
+#pragma unroll
+    for (int v = 0; v < kV; v++) T[v] = F[v] = 0;
+    for (int64_t base = 0; base < n; base += 1024)
+#pragma unroll
+        for (int v = 0; v < kV; v++) {
+            const int64_t k = base + v * NT + t;
+            if (k >= n) continue;
+            T[v] = join(T[v], read(2 * k));
+            F[v] += read(2 * k + 1);
+        }
+#pragma unroll
+    for (int h = kV / 2; h >= 1; h >>= 1)
+#pragma unroll
+        for (int v = 0; v < h; v++) {
+            T[v] = join(T[v], T[v + h]);
+            F[v] += F[v + h];
+        }
+    st[t] = T[0];
+    sg[t] = F[0];
+    __syncthreads();
+    for (int s = NT / 2; s >= 1; s >>= 1) {
+        if (t < s) {
+            st[t] = join(st[t], st[t + s]);
+            sg[t] += sg[t + s];
+        }
+        __syncthreads();
+    }
+    if (t == 0) {
+        out->theta = st[0];
+        out->gff = sg[0];
+    }
+}
+
+__global__ __launch_bounds__(1024) void k_reduce_quality(const double *partial, int64_t n, int crit_max,
+                                                         QualityResult *out)
+{
+    reduce_partials<1024, false>(partial, n, crit_max, out);
+}
+
+// SMALL: a lattice of at most one block per CU is bound by latency.  Its
+// eight links are loaded at once instead of two at a time, and with a.out the
+// block that finishes last reduces the partials (written and read coherently
+// at device scope, the count of finished blocks after a block's partials are
+// complete).  Larger lattices keep the second kernel: their blocks would
+// queue at the one count (FP32 32^4: 56 -> 79 us).  A whole check, FP64, the
+// result on the host: 8^4 24.1 -> 21.3 us, 16^4 25.1 -> 23.6 us; with the
+// second kernel, which no longer needs a copy after it, 24^4 44.8 -> 43.0 us,
+// 32^4 101.8 -> 101.3 us.
+template <typename R, int G, int S, bool SMALL>
 __global__ __launch_bounds__(kBlock) void k_quality(QualityArgs<R> a)
 {
     const int64_t L = ordered_block(a.order, blockIdx.x);
@@ -438,7 +504,7 @@ __global__ __launch_bounds__(kBlock) void k_quality(QualityArgs<R> a)
     double th = 0, gf = 0;
     if (active) {
         const int64_t site = p + (par ? a.g.Vh : 0);
-        quality_site<R, G, S>(a, site, th, gf);
+        quality_site<R, G, S, SMALL>(a, site, th, gf);
         if (a.dGff) {
             a.dGff[site] = gf;
             a.dA[site] = th;
@@ -459,14 +525,32 @@ __global__ __launch_bounds__(kBlock) void k_quality(QualityArgs<R> a)
         sh[1][wv] = gs;
     }
     __syncthreads();
+    __shared__ bool last;
     if (threadIdx.x == 0) {
         double T = sh[0][0], Gs = sh[1][0];
         for (int k = 1; k < kBlock / 64; k++) {
             T = a.crit_max ? fmax(T, sh[0][k]) : T + sh[0][k];
             Gs += sh[1][k];
         }
-        a.partial[2 * L] = T;
-        a.partial[2 * L + 1] = Gs;
+        if (SMALL && a.out) {
+            uint64_t *const o = (uint64_t *)a.partial + 2 * L;
+            __hip_atomic_store(o, (uint64_t)__double_as_longlong(T), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(o + 1, (uint64_t)__double_as_longlong(Gs), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the partials are complete
+            last = __hip_atomic_fetch_add(a.finished, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.order.n - 1;
+        } else {
+            a.partial[2 * L] = T;
+            a.partial[2 * L + 1] = Gs;
+        }
+    }
+    if constexpr (SMALL) {
+        if (!a.out) return;
+        __syncthreads();
+        if (!last) return;
+        // every block has counted: the next launch on these words starts at 0
+        if (threadIdx.x == 0) __hip_atomic_store(a.finished, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        reduce_partials<kBlock, true>(a.partial, a.order.n, a.crit_max, a.out);
     }
 }
 
@@ -478,11 +562,20 @@ static hipError_t launch_quality_s(int gauge, QualityArgs<R> a, hipStream_t s)
     static_assert(2 * kQualitySites == kBlock, "a block holds both parities' sites");
     a.order = make_block_order(quality_blocks(a.g.V), a.g.N[0], a.tpass);
     const unsigned grid = (unsigned)order_grid(a.order);
-    switch (gauge) {
-    case GF_COULOMB: hipLaunchKernelGGL((k_quality<R, GF_COULOMB, S>), dim3(grid), dim3(kBlock), 0, s, a); break;
-    case GF_MAG: hipLaunchKernelGGL((k_quality<R, GF_MAG, S>), dim3(grid), dim3(kBlock), 0, s, a); break;
-    default: hipLaunchKernelGGL((k_quality<R, GF_LANDAU, S>), dim3(grid), dim3(kBlock), 0, s, a); break;
-    }
+    const bool small = a.order.n <= 256;
+    const auto launch = [&](auto G_, auto SMALL_) {
+        constexpr int G = decltype(G_)::value;
+        hipLaunchKernelGGL((k_quality<R, G, S, decltype(SMALL_)::value>), dim3(grid), dim3(kBlock), 0, s, a);
+    };
+    const auto sized = [&](auto G_) {
+        if (small) launch(G_, std::true_type());
+        else launch(G_, std::false_type());
+    };
+    if (gauge == GF_COULOMB) sized(std::integral_constant<int, GF_COULOMB>());
+    else if (gauge == GF_MAG) sized(std::integral_constant<int, GF_MAG>());
+    else sized(std::integral_constant<int, GF_LANDAU>());
+    if (a.out && !small)
+        hipLaunchKernelGGL(k_reduce_quality, dim3(1), dim3(1024), 0, s, a.partial, (int64_t)a.order.n, a.crit_max, a.out);
     return hipGetLastError();
 }
 

@@ -76,11 +76,18 @@ inline int64_t kept_links(int64_t Vh, int64_t bytes)
     return (int64_t)((double)(4 * Vh) * (double)kKeptBytes / (double)bytes);
 }
 
+// A quality check's result, in host memory that the device maps.
+struct QualityResult {
+    double theta, gff;
+};
+
 template <typename R> struct QualityArgs {
     const R *U;
     Geom g;
     double *dGff, *dA;  // optional per-site outputs (V doubles each)
     double *partial;    // optional per-block (theta, gff) partials
+    QualityResult *out;  // optional, with partial: the lattice's theta and gff, reduced from the partials
+    uint32_t *finished;  // with out: a word that is 0, and 0 again after the launch (counts finished blocks)
     int crit_max;
     // a block takes the sites of both parities with parity-split index in
     // [128 L, 128 L + 128) (256 consecutive sites of the lexicographic order)
@@ -228,7 +235,6 @@ hipError_t launch_sweep(int stride, int gauge, int theta, bool gacc, const Sweep
 // utility kernels (su3gf_kernels.hip)
 hipError_t launch_convert(int ti, int si, const void *src, int to, int so, void *dst, int64_t V, int reun,
                           hipStream_t s);
-hipError_t launch_reduce_final(const double *partial, int64_t n, int crit_max, double *out, hipStream_t s);
 hipError_t launch_gauge_identity(float *g, int64_t V, hipStream_t s);
 hipError_t launch_project_gauge(float *g, int64_t V, hipStream_t s);
 // out_mu(x) = G(x) U0_mu(x) G(x+mu)^dagger with G = FP64 projection of g(x);

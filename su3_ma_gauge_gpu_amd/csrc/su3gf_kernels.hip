@@ -1,5 +1,4 @@
-// su3gf_kernels.hip -- utility kernels: layout/precision conversion, the
-// final fixed-order reduction of quality partials, and the gauge-transformation
+// su3gf_kernels.hip -- utility kernels: layout/precision conversion and the gauge-transformation
 // kernels of the mixed-precision driver (identity, reprojection, and the FP64
 // application out_mu(x) = G(x) U0_mu(x) G(x+mu)^dagger).
 #include "su3gf_sweep.h"
@@ -66,39 +65,6 @@ hipError_t launch_convert(int ti, int si, const void *src, int to, int so, void 
     if (ti == GF_F64 && to == GF_F32) return launch_convert_t(si, so, (const double *)src, (float *)dst, V, reun, s);
     if (ti == GF_F32 && to == GF_F64) return launch_convert_t(si, so, (const float *)src, (double *)dst, V, reun, s);
     return launch_convert_t(si, so, (const float *)src, (float *)dst, V, reun, s);
-}
-
-// ---------------------------------------------------------- final reduction
-// Fixed-order reduction of block partials: thread k sums partials k, k+1024,
-// ... in order, then a fixed tree -> out[0] = theta, out[1] = gff.
-__global__ __launch_bounds__(1024) void k_reduce_final(const double *partial, int64_t n, int crit_max, double *out)
-{
-    __shared__ double st[1024], sg[1024];
-    double T = 0, Gs = 0;
-    for (int64_t k = threadIdx.x; k < n; k += 1024) {
-        T = crit_max ? fmax(T, partial[2 * k]) : T + partial[2 * k];
-        Gs += partial[2 * k + 1];
-    }
-    st[threadIdx.x] = T;
-    sg[threadIdx.x] = Gs;
-    __syncthreads();
-    for (int s = 512; s >= 1; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            st[threadIdx.x] = crit_max ? fmax(st[threadIdx.x], st[threadIdx.x + s]) : st[threadIdx.x] + st[threadIdx.x + s];
-            sg[threadIdx.x] += sg[threadIdx.x + s];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        out[0] = st[0];
-        out[1] = sg[0];
-    }
-}
-
-hipError_t launch_reduce_final(const double *partial, int64_t n, int crit_max, double *out, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(1024), 0, s, partial, n, crit_max, out);
-    return hipGetLastError();
 }
 
 // ------------------------------------------------- gauge transformations
