@@ -123,8 +123,7 @@ inline hipStream_t S(void *stream) { return (hipStream_t)stream; }
 
 // Driver scratch memory, stream-ordered: allocated and freed on the driver's
 // stream (hipMallocAsync / hipFreeAsync), so a driver neither waits for nor
-// stalls work that other streams run meanwhile, and repeated runs reuse the
-// pool instead of the device allocator.
+// stalls work that other streams run meanwhile.
 struct Scratch {
     void *p = nullptr;
     hipStream_t s = nullptr;
@@ -143,23 +142,53 @@ struct Scratch {
     template <typename T> T *as() const { return (T *)p; }
 };
 
+// A run's buffers in one allocation: add() each, alloc() once, at() each.
+// The pool returns freed memory to the device at the next synchronisation, so
+// each run maps and unmaps anew, once for each allocation: allocating and freeing a mixed run's five, and
+// synchronising, takes 188 us at 12^4, 962 at 24^4 and 1274 at 48^4; one of
+// their total size takes 64, 338 and 698.
+struct RunScratch {
+    Scratch mem;
+    size_t bytes = 0;
+    size_t add(size_t n)
+    {
+        const size_t at = bytes;
+        bytes += (n + 4095) / 4096 * 4096;
+        return at;
+    }
+    hipError_t alloc(hipStream_t s) { return bytes ? mem.alloc(bytes, s) : hipSuccess; }
+    template <typename T> T *at(size_t offset) const { return (T *)((char *)mem.p + offset); }
+};
+
 // The synchronisation words of a lattice's pipelined sweeps
 // (launch_gsweep_pipe), allocated and zeroed only where that sweep applies.
 // check() reports a dependency wait that ran out of its spin limit.
 struct PipeBuf {
-    Scratch mem;
+    Scratch mem;  // of init
+    PipeSync *words = nullptr;
     uint32_t count = 0;  // launches on these words (block-index order)
+    static size_t bytes(const Geom &geo, int gauge, bool links64)
+    {
+        if (!gsweep_pipe_applies(geo, gauge, links64)) return 0;
+        return sizeof(uint32_t) * pipe_sync_words(sweep_grid(geo));
+    }
+    // n = bytes(...) bytes of the caller's
+    hipError_t init_at(void *p, size_t n, hipStream_t s)
+    {
+        if (!n) return hipSuccess;
+        words = (PipeSync *)p;
+        return hipMemsetAsync(p, 0, n, s);
+    }
     hipError_t init(const Geom &geo, int gauge, bool links64, hipStream_t s)
     {
-        if (!gsweep_pipe_applies(geo, gauge, links64)) return hipSuccess;
-        const size_t bytes = sizeof(uint32_t) * pipe_sync_words(sweep_grid(geo));
-        const hipError_t e = mem.alloc(bytes, s);
-        return e != hipSuccess ? e : hipMemsetAsync(mem.p, 0, bytes, s);
+        const size_t n = bytes(geo, gauge, links64);
+        const hipError_t e = n ? mem.alloc(n, s) : hipSuccess;
+        return e != hipSuccess ? e : init_at(mem.p, n, s);
     }
-    PipeSync *get() const { return mem.as<PipeSync>(); }
+    PipeSync *get() const { return words; }
     gf_status check(hipStream_t s) const
     {
-        if (!mem.p) return GF_OK;
+        if (!words) return GF_OK;
         uint32_t err = 0;
         if (hipMemcpyAsync(&err, &get()->err, sizeof err, hipMemcpyDeviceToHost, s) != hipSuccess ||
             hipStreamSynchronize(s) != hipSuccess)
@@ -1084,25 +1113,28 @@ extern "C" gf_status gf_run_sa(const gf_lattice *lat, void *U, void *Udw, int ga
     gf_lattice l32 = *lat;
     l32.dtype = GF_F32;
     l32.layout = GF_LAYOUT_R12;
-    Scratch bU32, bg;
+    RunScratch mem;
     PipeBuf pipe;
     GaugeSweepArgs ga{};
     const Geom geo = make_geom(lat->dims, V);
     if (gform) {
-        HIP_TRY(bU32.alloc(mode == 2 ? sizeof(uint32_t) * links24_words(V) : gf_lattice_bytes(&l32), s));
-        HIP_TRY(bg.alloc(sizeof(float) * gauge_floats(V), s));
-        HIP_TRY(launch_gauge_identity(bg.as<float>(), V, s));
-        if (mode == 2) HIP_TRY(launch_pack24(lat->dtype, lat->layout, U, bU32.as<uint32_t>(), V, s));
-        else HIP_TRY(launch_convert(lat->dtype, lat->layout, U, GF_F32, 12, bU32.p, V, 0, s));
+        const size_t oU = mem.add(mode == 2 ? sizeof(uint32_t) * links24_words(V) : gf_lattice_bytes(&l32));
+        const size_t og = mem.add(sizeof(float) * gauge_floats(V));
+        // (a captured schedule keeps the two-kernel sweeps: the pipelined
+        // sweep's launch numbers come from the host at each launch)
+        const size_t npipe = graph ? 0 : PipeBuf::bytes(geo, gauge, false);
+        const size_t opipe = mem.add(npipe);
+        HIP_TRY(mem.alloc(s));
+        ga.U0 = mem.at<float>(oU);
+        ga.g = mem.at<float>(og);
+        HIP_TRY(launch_gauge_identity(ga.g, V, s));
+        if (mode == 2) HIP_TRY(launch_pack24(lat->dtype, lat->layout, U, mem.at<uint32_t>(oU), V, s));
+        else HIP_TRY(launch_convert(lat->dtype, lat->layout, U, GF_F32, 12, mem.at<void>(oU), V, 0, s));
+        HIP_TRY(pipe.init_at(mem.at<void>(opipe), npipe, s));
         ga.links24 = mode == 2;
-        ga.U0 = bU32.as<const float>();
-        ga.g = bg.as<float>();
         ga.geo = geo;
         ga.seed = (uint32_t)seed;
         ga.nsb = 32;
-        // (a captured schedule keeps the two-kernel sweeps: the pipelined
-        // sweep's launch numbers come from the host at each launch)
-        if (!graph) HIP_TRY(pipe.init(geo, gauge, false, s));
         ga.pipe = pipe.get();
         ga.pipe_count = &pipe.count;
     }
@@ -1151,9 +1183,8 @@ extern "C" gf_status gf_run_sa(const gf_lattice *lat, void *U, void *Udw, int ga
     if (graph) GF_TRY(gr.replay());
     if (gform) {
         // U <- G U G^dagger in FP64 (G the FP64 projection of g), third rows rebuilt
-        HIP_TRY(launch_project_gauge(bg.as<float>(), V, s));
-        HIP_TRY(launch_gauge_apply((const double *)U, lat->layout, bg.as<const float>(), U, GF_F64, lat->layout, geo,
-                                   s));
+        HIP_TRY(launch_project_gauge(ga.g, V, s));
+        HIP_TRY(launch_gauge_apply((const double *)U, lat->layout, ga.g, U, GF_F64, lat->layout, geo, s));
         GF_TRY(gf_project(lat, U, s));
         HIP_TRY(hipStreamSynchronize(s));
         GF_TRY(pipe.check(s));
@@ -1174,24 +1205,30 @@ gf_status run_sa_multi(const int *idx, int n, const gf_lattice *lats, void *cons
                        int steps, int micro, int mode, bool graph, const int *seeds, uint32_t *counters,
                        int *temperatures, hipStream_t s)
 {
-    Scratch bU[kMultiMax], bg[kMultiMax];
+    RunScratch mem;
+    size_t oU[kMultiMax], og[kMultiMax];
     MultiSweepArgs m{};
     m.n = n;
+    for (int j = 0; j < n; j++) {
+        int64_t V;
+        GF_TRY(check_lattice(&lats[idx[j]], &V));
+        gf_lattice l32 = lats[idx[j]];
+        l32.dtype = GF_F32;
+        l32.layout = GF_LAYOUT_R12;
+        oU[j] = mem.add(mode == 2 ? sizeof(uint32_t) * links24_words(V) : gf_lattice_bytes(&l32));
+        og[j] = mem.add(sizeof(float) * gauge_floats(V));
+    }
+    HIP_TRY(mem.alloc(s));
     for (int j = 0; j < n; j++) {
         const int k = idx[j];
         const gf_lattice *lat = &lats[k];
         int64_t V;
         GF_TRY(check_lattice(lat, &V));
-        gf_lattice l32 = *lat;
-        l32.dtype = GF_F32;
-        l32.layout = GF_LAYOUT_R12;
-        HIP_TRY(bU[j].alloc(mode == 2 ? sizeof(uint32_t) * links24_words(V) : gf_lattice_bytes(&l32), s));
-        HIP_TRY(bg[j].alloc(sizeof(float) * gauge_floats(V), s));
-        HIP_TRY(launch_gauge_identity(bg[j].as<float>(), V, s));
-        if (mode == 2) HIP_TRY(launch_pack24(lat->dtype, lat->layout, U[k], bU[j].as<uint32_t>(), V, s));
-        else HIP_TRY(launch_convert(lat->dtype, lat->layout, U[k], GF_F32, 12, bU[j].p, V, 0, s));
-        m.item[j] = MultiItem{bU[j].as<const float>(), bg[j].as<float>(), make_geom(lat->dims, V), (uint32_t)seeds[k],
-                              counters[k]};
+        float *const g = mem.at<float>(og[j]);
+        HIP_TRY(launch_gauge_identity(g, V, s));
+        if (mode == 2) HIP_TRY(launch_pack24(lat->dtype, lat->layout, U[k], mem.at<uint32_t>(oU[j]), V, s));
+        else HIP_TRY(launch_convert(lat->dtype, lat->layout, U[k], GF_F32, 12, mem.at<void>(oU[j]), V, 0, s));
+        m.item[j] = MultiItem{mem.at<float>(oU[j]), g, make_geom(lat->dims, V), (uint32_t)seeds[k], counters[k]};
     }
     uint32_t add = 0;  // every lattice's counter advances by 2 per heatbath step, as in gf_run_sa
     auto pair = [&](int algo) -> hipError_t {
@@ -1220,9 +1257,8 @@ gf_status run_sa_multi(const int *idx, int n, const gf_lattice *lats, void *cons
         const int k = idx[j];
         const gf_lattice *lat = &lats[k];
         const Geom &geo = m.item[j].geo;
-        HIP_TRY(launch_project_gauge(bg[j].as<float>(), geo.V, s));
-        HIP_TRY(launch_gauge_apply((const double *)U[k], lat->layout, bg[j].as<const float>(), U[k], GF_F64,
-                                   lat->layout, geo, s));
+        HIP_TRY(launch_project_gauge(m.item[j].g, geo.V, s));
+        HIP_TRY(launch_gauge_apply((const double *)U[k], lat->layout, m.item[j].g, U[k], GF_F64, lat->layout, geo, s));
         GF_TRY(gf_project(lat, U[k], s));
         counters[k] += add;
         if (temperatures) temperatures[k] = nt;
@@ -1322,7 +1358,8 @@ namespace {
 constexpr size_t fused_scratch_bytes(int64_t blocks) { return 256 + sizeof(double) * 4 * (size_t)blocks; }
 
 struct FusedCtx {
-    Scratch dev;                // DevState, then 2 * nblocks doubles for each parity
+    Scratch dev;                // of init
+    // one buffer holds DevState, then 2 * nblocks doubles for each parity
     DevState *st = nullptr;     // device
     DevState *host = nullptr;   // pinned, or own_host
     DevState own_host;          // the allocation-free driver's (pageable) copy
@@ -1332,15 +1369,17 @@ struct FusedCtx {
     int64_t nblocks = 0;
     gf_status init(int64_t blocks, hipStream_t s)  // partial sums for up to `blocks` blocks per parity
     {
-        nblocks = blocks;
-        HIP_TRY(dev.alloc(fused_scratch_bytes(nblocks), s));  // state, even, odd
-        st = dev.as<DevState>();
-        partial = (double *)((char *)dev.p + 256);
+        HIP_TRY(dev.alloc(fused_scratch_bytes(blocks), s));
+        return init_in(dev.p, blocks);
+    }
+    // in fused_scratch_bytes(blocks) bytes of the caller's device memory
+    gf_status init_in(void *mem, int64_t blocks)
+    {
+        init_at(mem, blocks);
         HIP_TRY(pinned_state(&host));
         return GF_OK;
     }
-    // the same layout in caller-provided device memory (fused_scratch_bytes(blocks)
-    // bytes); the host copy of the state is this object's own
+    // the same, with the host copy of the state this object's own
     void init_at(void *mem, int64_t blocks)
     {
         nblocks = blocks;
@@ -1557,16 +1596,21 @@ gf_status project_unless_done(const gf_lattice *lat, void *U, const DevState *st
 // (kTiled12): a block's 64 sites then read and write one contiguous 6 KB
 // tile per direction instead of twelve 512-byte pieces V * 8 bytes apart.
 struct Tiles64 {
-    Scratch buf;
+    Scratch buf;  // of init
     gf_lattice lat{};
     double *p = nullptr;
     gf_status init(const gf_lattice *caller, int64_t V, hipStream_t s)
     {
+        HIP_TRY(buf.alloc(bytes(V), s));
+        init_at(caller, buf.p);
+        return GF_OK;
+    }
+    static size_t bytes(int64_t V) { return sizeof(double) * 4 * tiled12_reals(V); }
+    void init_at(const gf_lattice *caller, void *mem)
+    {
         lat = *caller;
         lat.layout = kTiled12;
-        HIP_TRY(buf.alloc(sizeof(double) * 4 * tiled12_reals(V), s));
-        p = buf.as<double>();
-        return GF_OK;
+        p = (double *)mem;
     }
 };
 
@@ -1624,11 +1668,15 @@ gf_status gf_run_fast(const gf_lattice *lat, void *U, int gauge, float omega, fl
         return fail(GF_ERR_BAD_ARG, "FP32 fused sweeps work on the compact 12-real layout");
     memset(out, 0, sizeof *out);
     hipStream_t s = S(stream);
-    FusedCtx fc;
-    GF_TRY(fc.init(sweep_grid(per_slice(make_geom(lat->dims, V), gauge)), s));
-    Tiles64 tiles;
     const bool f64 = lat->dtype == GF_F64;
-    if (f64) GF_TRY(tiles.init(lat, V, s));
+    const int64_t blocks = sweep_grid(per_slice(make_geom(lat->dims, V), gauge));
+    RunScratch mem;
+    const size_t ofc = mem.add(fused_scratch_bytes(blocks)), otiles = mem.add(f64 ? Tiles64::bytes(V) : 0);
+    HIP_TRY(mem.alloc(s));
+    FusedCtx fc;
+    GF_TRY(fc.init_in(mem.at<void>(ofc), blocks));
+    Tiles64 tiles;
+    if (f64) tiles.init_at(lat, mem.at<void>(otiles));
     EventPair ev;
     HIP_TRY(hipEventCreate(&ev.a));
     HIP_TRY(hipEventCreate(&ev.b));
@@ -1834,24 +1882,28 @@ gf_status gf_run_mixed(const gf_lattice *lat, void *U, int gauge, float omega, f
     l32.dtype = GF_F32;
     l32.layout = GF_LAYOUT_R12;
     const Geom geo = per_slice(make_geom(lat->dims, V), gauge);
-    Scratch sU32, sg, sg64;
+    RunScratch mem;
+    size_t oU32 = 0, og = 0, og64 = 0, npipe = 0, opipe = 0;
     if (fp32_phase) {
-        HIP_TRY(sU32.alloc(mode == GF_MIXED_GAUGE24 ? sizeof(uint32_t) * links24_words(V) : gf_lattice_bytes(&l32),
-                           s));
-        HIP_TRY(sg.alloc(sizeof(float) * gauge_floats(V), s));
+        oU32 = mem.add(mode == GF_MIXED_GAUGE24 ? sizeof(uint32_t) * links24_words(V) : gf_lattice_bytes(&l32));
+        og = mem.add(sizeof(float) * gauge_floats(V));
+        if (mode != GF_MIXED_LINKS) npipe = PipeBuf::bytes(geo, gauge, false);
+        opipe = mem.add(npipe);
     }
     // the gauge modes' FP64 phase sweeps an FP64 g on the FP64 links (the
     // link mode, and lattices beyond the FP64 gauge sweep's offsets, sweep
     // the links themselves)
     const bool gauge64 = mode != GF_MIXED_LINKS && gauge_sweep64_fits(V);
-    if (gauge64) HIP_TRY(sg64.alloc(sizeof(double) * gauge_floats(V), s));
+    if (gauge64) og64 = mem.add(sizeof(double) * gauge_floats(V));
+    const size_t ofc = mem.add(fused_scratch_bytes(sweep_grid(geo))), otiles = mem.add(Tiles64::bytes(V));
+    HIP_TRY(mem.alloc(s));
     struct {
         void *U32, *g;
-    } b{sU32.p, sg.p};
+    } b{mem.at<void>(oU32), mem.at<void>(og)};  // of the FP32 phase
     FusedCtx fc;
-    GF_TRY(fc.init(sweep_grid(geo), s));
+    GF_TRY(fc.init_in(mem.at<void>(ofc), sweep_grid(geo)));
     Tiles64 tiles;  // the FP64 phase's links
-    GF_TRY(tiles.init(lat, V, s));
+    tiles.init_at(lat, mem.at<void>(otiles));
     EventPair ev;
     hipEvent_t mid = nullptr;
     HIP_TRY(hipEventCreate(&ev.a));
@@ -1897,7 +1949,7 @@ gf_status gf_run_mixed(const gf_lattice *lat, void *U, int gauge, float omega, f
         ga.param = omega;
         ga.links24 = mode == GF_MIXED_GAUGE24;
         PipeBuf pipe;
-        HIP_TRY(pipe.init(geo, gauge, false, s));
+        HIP_TRY(pipe.init_at(mem.at<void>(opipe), npipe, s));
         ga.pipe = pipe.get();
         ga.pipe_count = &pipe.count;
         auto launch = [&](int parity, int theta, double *partial, int) {
@@ -1977,7 +2029,7 @@ gf_status gf_run_mixed(const gf_lattice *lat, void *U, int gauge, float omega, f
         // links G U0 G^dagger, read only: the same OR updates as sweeping the
         // links, with 1056 instead of 1536 bytes per site-update; g64 is
         // re-orthonormalised in every update, so nothing is reprojected
-        double *g64 = sg64.as<double>();
+        double *g64 = mem.at<double>(og64);
         HIP_TRY(launch_gauge_identity64(g64, V, s));
         GaugeSweepArgs gd{};
         gd.U0 = (const float *)tiles.p;
