@@ -340,15 +340,18 @@ gf_status gf_set_pipelined_lag(int lag, int *previous);
  * it with t innermost, so that a block's t neighbours were read by the block
  * before it.  Walking the range in passes of n timeslices brings a block's x
  * neighbours closer in that sequence, at the cost of the t neighbours across
- * a pass boundary.  The results do not depend on the order (the sites of a
- * parity are independent); the time does.  Chosen per lattice shape, gauge
- * and mode by timing, together with the wavefront slab.
+ * a pass boundary.  Where Nt is no multiple of 8, groups of n timeslices are
+ * walked instead, n a divisor of Nt (up to 8 by default), and each XCD takes
+ * an eighth of that sequence.  The results do not depend on the order (the
+ * sites of a parity are independent); the time does.  Chosen per lattice
+ * shape, gauge and mode by timing, together with the wavefront slab.
  * The drop-in quality kernel (gf_stats_quality, gf_quality_per_site) walks
  * the XCDs' timeslices the same way, and its order is tuned on its first
  * launch for a kind of lattice (timing launches read the links and write
  * nothing), under the same setting.
- * gf_set_block_order: -1 choose by timing (default), 0 one pass, n > 0 passes
- * of n timeslices (where n divides the XCD's range; otherwise one pass);
+ * gf_set_block_order: -1 choose by timing (default), 0 one pass (or the
+ * default groups), n > 0 passes of n timeslices (where n divides the XCD's
+ * range, or Nt if it is no multiple of 8; otherwise as 0);
  * *previous (optional) receives the old setting.
  * gf_block_order_choice: the order in use for gf_run_mixed of lat with
  * `gauge` and gauge-sweep `mode` (-1 not chosen yet).

@@ -17,7 +17,8 @@
 // kernels each direction's combined share -- so the four waves hold
 // bit-identical sums and compute the same update, which each lane applies to
 // its own two links.  Two LDS buffers alternate between subgroups, so one
-// barrier per subgroup suffices.
+// barrier per subgroup suffices.  The updates that draw random numbers have a
+// kernel of their own (k_sweep_rng, su3gf_exact.hip).
 //
 // Reference (paths relative to its src/): GaugeFixingSubgroupStep.hxx:74-705,
 // algorithms/{Or,Micro,Sa,Sr,Random}Update.hxx, {Landau,Coulomb,MAG,U1xU1}KernelsSU3.hxx
