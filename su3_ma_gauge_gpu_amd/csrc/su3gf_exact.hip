@@ -538,7 +538,7 @@ __global__ __launch_bounds__(kBlock) void k_quality(QualityArgs<R> a)
             __hip_atomic_store(o + 1, (uint64_t)__double_as_longlong(Gs), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
             __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the partials are complete
-            last = __hip_atomic_fetch_add(a.finished, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.order.n - 1;
+            last = atomicInc(a.finished, a.order.n - 1) == a.order.n - 1;  // (wraps to 0 for the next launch)
         } else {
             a.partial[2 * L] = T;
             a.partial[2 * L + 1] = Gs;
@@ -548,8 +548,6 @@ __global__ __launch_bounds__(kBlock) void k_quality(QualityArgs<R> a)
         if (!a.out) return;
         __syncthreads();
         if (!last) return;
-        // every block has counted: the next launch on these words starts at 0
-        if (threadIdx.x == 0) __hip_atomic_store(a.finished, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         reduce_partials<kBlock, true>(a.partial, a.order.n, a.crit_max, a.out);
     }
 }
