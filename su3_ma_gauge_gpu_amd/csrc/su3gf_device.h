@@ -455,30 +455,4 @@ __device__ __forceinline__ void philox_at(uint32_t k0, uint32_t k1, uint32_t c1,
     for (int k = 0; k < 4; k++) u[k] = (float)(1 + (w[k] >> 8)) * 0x1.fffffep-25f;
 }
 
-// ------------------------------------------------------ quad reductions
-// The four lanes of a quad hold the four directions of one site.  A butterfly
-// over quad_perm [1,0,3,2] then [2,3,0,1] leaves the same, bit-identical sum
-// in all four lanes (floating-point addition is commutative).
-template <int CTRL> __device__ __forceinline__ float dpp(float v)
-{
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
-}
-template <int CTRL> __device__ __forceinline__ double dpp(double v)
-{
-    const int64_t b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_mov_dpp((int)(b & 0xffffffff), CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, false);
-    return __longlong_as_double(((int64_t)hi << 32) | (uint32_t)lo);
-}
-
-constexpr int QP_XOR1 = 0xB1;  // quad_perm [1,0,3,2]
-constexpr int QP_XOR2 = 0x4E;  // quad_perm [2,3,0,1]
-
-template <typename R> __device__ __forceinline__ R quad_sum(R v)
-{
-    v = v + dpp<QP_XOR1>(v);
-    v = v + dpp<QP_XOR2>(v);
-    return v;
-}
-
 }  // namespace su3gf
