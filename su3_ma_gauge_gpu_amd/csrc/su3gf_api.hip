@@ -255,7 +255,8 @@ struct gf_stats {
     int64_t V;
     int64_t nblocks;
     double *partial;       // device, 2 * nblocks
-    uint32_t *finished;    // device, 1: the quality kernel's count of finished blocks, 0 between calls
+    uint32_t *finished;    // device, 1: the quality kernel's count of finished blocks, 0 between checks
+    bool counted;          // a check has run: finished holds its 0
     QualityResult *host;   // pinned host, written by the kernel
 };
 
@@ -514,7 +515,6 @@ gf_status gf_stats_create(const int dims[4], int gauge, int crit, gf_stats **out
     st->nblocks = exact::quality_blocks(V);
     hipError_t e = hipMalloc((void **)&st->partial, sizeof(double) * 2 * st->nblocks);
     if (e == hipSuccess) e = hipMalloc((void **)&st->finished, sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMemset(st->finished, 0, sizeof(uint32_t));
     if (e == hipSuccess) e = hipHostMalloc((void **)&st->host, sizeof(QualityResult), hipHostMallocCoherent);
     if (e != hipSuccess) {
         if (st->partial) (void)hipFree(st->partial);
@@ -584,8 +584,12 @@ gf_status gf_stats_quality(gf_stats *st, const gf_lattice *lat, const void *U, d
     for (int i = 0; i < 4; i++)
         if (lat->dims[i] != st->dims[i]) return fail(GF_ERR_BAD_SHAPE, "lattice shape differs from the stats shape");
     const int crit_max = st->crit == GF_CRIT_MAX;
+    // the first check zeroes the count on its own stream (the caller's need not
+    // wait for the null stream, nor for a fill made when the handle was)
+    if (!st->counted) HIP_TRY(hipMemsetAsync(st->finished, 0, sizeof(uint32_t), S(stream)));
     GF_TRY(quality_launch(lat, st->gauge, U, nullptr, nullptr, st->partial, st, crit_max, S(stream)));
     HIP_TRY(hipStreamSynchronize(S(stream)));
+    st->counted = true;
     // GaugeFixingStats.hxx:203-206 with the per-gauge prefactors
     const double Nc = 3.0, Ndim = 4.0;
     const double pg = st->gauge == GF_COULOMB ? 1. / (Nc * (Ndim - 1)) : 1. / (Nc * Ndim);
