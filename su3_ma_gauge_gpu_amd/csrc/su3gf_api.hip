@@ -13,6 +13,7 @@
 #include <array>
 #include <map>
 #include <chrono>
+#include <limits>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -584,6 +585,8 @@ gf_status gf_stats_quality(gf_stats *st, const gf_lattice *lat, const void *U, d
     for (int i = 0; i < 4; i++)
         if (lat->dims[i] != st->dims[i]) return fail(GF_ERR_BAD_SHAPE, "lattice shape differs from the stats shape");
     const int crit_max = st->crit == GF_CRIT_MAX;
+    // a check that leaves no result reports NaN, not the one before it
+    st->host->theta = st->host->gff = std::numeric_limits<double>::quiet_NaN();
     // the first check zeroes the count on its own stream (the caller's need not
     // wait for the null stream, nor for a fill made when the handle was)
     if (!st->counted) HIP_TRY(hipMemsetAsync(st->finished, 0, sizeof(uint32_t), S(stream)));

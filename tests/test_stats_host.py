@@ -30,3 +30,9 @@ def test_count_is_zero_on_the_checks_own_stream(counts):
     assert counts["launches"] == 3 and counts["words"] == 1
     assert counts["unordered"] == 0
     assert counts["not_zero"] == 0
+
+
+def test_a_check_without_a_result_reports_none(counts):
+    """Where the kernel leaves no result, theta and gff are NaN: not what the
+    memory held, nor the check's before it."""
+    assert counts["stale"] == 0
