@@ -1135,66 +1135,40 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_mag(GaugeSweepArgs a)
 // products w w^dagger of column c of W over the eight links: for the subgroup
 // (i, j) D = (P_i - P_j)_ii - (P_i - P_j)_jj and c = (P_i - P_j)_ij, theta_x's
 // X_ij is that c, and the functional's sum of |U_jj|^2 is the sum of (P_j)_jj.
-// W is unitary, so P_2 = 8 - P_0 - P_1, and only columns 0 and 1 are formed.
-// Wave mu forms its two links' columns without g(x) -- of U0_mu(x) g(y)^dagger,
-// and rows 0, 1 of g(z) U0_mu(z), conjugated -- and their outer products, 18
-// reals that go through LDS; wave 0 adds the four, rotates the sums by g(x) and
-// makes the three updates on them (P_c <- G P_c G^dagger) and on g(x).  The
-// four waves thus stop after their products (about 370 of the 1220 to 1640
-// VALU instructions per wave of the sweep on the links themselves, as
-// k_gsweep_mag makes it, where every wave turns its links by g(x) and by the
-// three updates), with one barrier instead of six: 24^4 42.6 -> 31.7 us per
-// checked launch, 32^4 130 -> 94, 48^4 687 -> 566, which is the Landau sweep's
-// time (31, 92, 559): the bytes bound it now.
+// Two differences give all of them: A = P_0 - P_2 and B = P_1 - P_2 (X_01 is
+// that of A - B), with the trace of P_2 for the functional.
+// Wave mu turns its two links by g(x), as the sweep on the links themselves
+// does, and forms their share of A, B and the trace, 19 reals that go through
+// LDS; wave 0 adds the four and makes the three updates on the sums
+// (P <- G P G^dagger) and on g(x).  The waves thus stop after their products
+// and do not turn their links by the three updates, with one barrier instead of
+// six: checked launch, with every link turned and as here, 12^4 8.8 and 7.6 us,
+// 24^4 42.5 and 33.1, 32^4 138 and 107, 40^4 342 and 271, 48^4 700 and 624.
+// Sums of links not yet turned by g(x), which wave 0 turns instead (columns 0
+// and 1 only, P_2 = 8 - P_0 - P_1 by unitarity), take 31, 95, 246 and 560 us at
+// 24^4 to 48^4, but they are of order 8 where the turned ones' off-diagonal
+// entries are small, and turning them cancels: theta then stops falling at
+// 2.0e-15, against 1.37e-15 for turned links, here as on the links themselves,
+// and links unitary to single precision are swept differently by 5e-7.
 template <typename A> struct Outer {
     A d[3];       // the diagonal
     Cx<A> o[3];   // (0,1), (0,2), (1,2)
 };
-// += w w^dagger
-template <typename A> __device__ __forceinline__ void add_outer(Outer<A> &P, const Cx<A> w[3])
+// += w w^dagger - v v^dagger
+template <typename A> __device__ __forceinline__ void add_outer(Outer<A> &P, const Cx<A> w[3], const Cx<A> v[3])
 {
 #pragma unroll
     for (int i = 0; i < 3; i++) {
         P.d[i] = fma_(w[i].x, w[i].x, P.d[i]);
         P.d[i] = fma_(w[i].y, w[i].y, P.d[i]);
-    }
-    cmacc(P.o[0], w[0], w[1]);
-    cmacc(P.o[1], w[0], w[2]);
-    cmacc(P.o[2], w[1], w[2]);
-}
-// P <- g P g^dagger
-template <typename A> __device__ __forceinline__ void turn(Outer<A> &P, const M3<A> &g)
-{
-    M3<A> T;  // g P
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        T.e[i][0] = g.e[i][0] * P.d[0];
-        cmacc(T.e[i][0], g.e[i][1], P.o[0]);
-        cmacc(T.e[i][0], g.e[i][2], P.o[1]);
-        T.e[i][1] = g.e[i][1] * P.d[1];
-        cmac(T.e[i][1], g.e[i][0], P.o[0]);
-        cmacc(T.e[i][1], g.e[i][2], P.o[2]);
-        T.e[i][2] = g.e[i][2] * P.d[2];
-        cmac(T.e[i][2], g.e[i][0], P.o[1]);
-        cmac(T.e[i][2], g.e[i][1], P.o[2]);
-    }
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        A d = 0;
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            d = fma_(T.e[i][k].x, g.e[i][k].x, d);
-            d = fma_(T.e[i][k].y, g.e[i][k].y, d);
-        }
-        P.d[i] = d;
+        P.d[i] = fma_(-v[i].x, v[i].x, P.d[i]);
+        P.d[i] = fma_(-v[i].y, v[i].y, P.d[i]);
     }
 #pragma unroll
     for (int m = 0; m < 3; m++) {
         const int i = m == 2 ? 1 : 0, j = m == 0 ? 1 : 2;
-        Cx<A> s = czero<A>();
-#pragma unroll
-        for (int k = 0; k < 3; k++) cmacc(s, T.e[i][k], g.e[j][k]);
-        P.o[m] = s;
+        cmacc(P.o[m], w[i], w[j]);
+        cmacc(P.o[m], cx(-v[i].x, -v[i].y), v[j]);
     }
 }
 // P <- G P G^dagger for the SU(2) element q of subgroup (I, J), whose q3 is 0:
@@ -1230,7 +1204,8 @@ template <int THETA, bool STREAM>
 __global__ __launch_bounds__(kGBlock) void k_gsweep_mag64(GaugeSweepArgs a)
 {
     using A = double;
-    __shared__ A lds[18 * 4 * 64];
+    constexpr int kVals = THETA ? 19 : 18;  // A, B and, for the functional, the trace of P_2
+    __shared__ A lds[kVals * 4 * 64];
     if (a.state && a.state->done) return;  // converged: uniform early exit
     if (THETA == 3 && !a.state->near) return;
     const int mu = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1258,44 +1233,47 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_mag64(GaugeSweepArgs a)
         kz = kept_link(a.keep, a.geo.Vh, par ? z : z - a.geo.Vh, mu);
     }
     M3<A> Gx;
-    if (mu == 0) {
-        if (stream_g) load_g<A, 2, kNt>(fg, site_off, Gx);
-        else load_g<A, 2>(fg, site_off, Gx);
-    }
+    if (stream_g) load_g<A, 2, kNt>(fg, site_off, Gx);
+    else load_g<A, 2>(fg, site_off, Gx);
+    Outer<A> P[2] = {};  // A, B
+    A tr = 0;
     {
-        Outer<A> P[2] = {};
-        M3<A> T, W;
+        // columns w[0..2] of one link
+        const auto add = [&](const Cx<A> (&w)[3][3]) {
+            add_outer(P[0], w[0], w[2]);
+            add_outer(P[1], w[1], w[2]);
+            if (THETA)
+#pragma unroll
+                for (int i = 0; i < 3; i++) {
+                    tr = fma_(w[2][i].x, w[2][i].x, tr);
+                    tr = fma_(w[2][i].y, w[2][i].y, tr);
+                }
+        };
+        M3<A> T, W, X;
+        Cx<A> w[3][3];
         const uint32_t y_off = site_boff<2>(forward(a.geo, c, par, mu)), z_off = site_boff<2>(z);
         const Field fu = links_field<2>(a.U0, a.geo.V, mu);
         load_links<A, 2, STREAM>(fu, site_off, W, kx);
         load_g<A, 2>(fg, y_off, T);
-        third_row(W);
+        third_row(T);
+        prod_adag(X, W, T);
+        third_row(Gx);
+        prod_ab(W, Gx, X);  // g(x) U0_mu(x) g(y)^dagger
 #pragma unroll
-        for (int k = 0; k < 2; k++) {  // column k of U0_mu(x) g(y)^dagger
-            Cx<A> w[3];
+        for (int k = 0; k < 3; k++)
 #pragma unroll
-            for (int i = 0; i < 3; i++) {
-                w[i] = czero<A>();
-#pragma unroll
-                for (int j = 0; j < 3; j++) cmacc(w[i], W.e[i][j], T.e[k][j]);
-            }
-            add_outer(P[k], w);
-        }
+            for (int i = 0; i < 3; i++) w[k][i] = W.e[i][k];
+        add(w);
         load_g<A, 2>(fg, z_off, T);
         load_links<A, 2, STREAM>(fu, z_off, W, kz);
         third_row(W);
+        prod_ab(X, T, W);
+        prod_adag(W, X, Gx);  // g(z) U0_mu(z) g(x)^dagger
 #pragma unroll
-        for (int k = 0; k < 2; k++) {  // row k of g(z) U0_mu(z), conjugated
-            Cx<A> w[3];
+        for (int k = 0; k < 3; k++)
 #pragma unroll
-            for (int i = 0; i < 3; i++) {
-                w[i] = czero<A>();
-#pragma unroll
-                for (int j = 0; j < 3; j++) cmac(w[i], T.e[k][j], W.e[j][i]);
-                w[i] = conj(w[i]);
-            }
-            add_outer(P[k], w);
-        }
+            for (int i = 0; i < 3; i++) w[k][i] = conj(W.e[k][i]);
+        add(w);
 #pragma unroll
         for (int k = 0; k < 2; k++)
 #pragma unroll
@@ -1305,28 +1283,26 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_mag64(GaugeSweepArgs a)
                 b[256] = P[k].o[i].x;
                 b[512] = P[k].o[i].y;
             }
+        if (THETA) lds[(kVals - 1) * 256 + mu * 64 + lane] = tr;
     }
     __syncthreads();
     if (mu != 0) return;
-    third_row(Gx);
-    Outer<A> P[2];
     const auto sum = [&](int v) {  // value v of the four directions, in the order of mu
         const A *const b = lds + v * 256 + lane;
         return ((b[0] + b[64]) + b[128]) + b[192];
     };
 #pragma unroll
-    for (int k = 0; k < 2; k++) {
+    for (int k = 0; k < 2; k++)
 #pragma unroll
         for (int i = 0; i < 3; i++) {
             P[k].d[i] = sum(9 * k + 3 * i);
             P[k].o[i] = cx(sum(9 * k + 3 * i + 1), sum(9 * k + 3 * i + 2));
         }
-        turn(P[k], Gx);
-    }
-    // the subgroups' c = X_ij, and D (P_2 = 8 - P_0 - P_1)
+    if (THETA) tr = sum(kVals - 1);
+    // the subgroups' c = X_ij, and D
     const auto x01 = [&] { return P[0].o[0] - P[1].o[0]; };
-    const auto x02 = [&] { return P[0].o[1] * (A)2 + P[1].o[1]; };
-    const auto x12 = [&] { return P[1].o[2] * (A)2 + P[0].o[2]; };
+    const auto x02 = [&] { return P[0].o[1]; };
+    const auto x12 = [&] { return P[1].o[2]; };
     const auto theta = [&]() {
         const Cx<A> x[3] = {x01(), x02(), x12()};
         double s[kThetaVals];
@@ -1335,7 +1311,7 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_mag64(GaugeSweepArgs a)
             s[2 * k] = x[k].x;
             s[2 * k + 1] = x[k].y;
         }
-        s[9] = (P[0].d[0] + P[1].d[1]) + ((A)8 - (P[0].d[2] + P[1].d[2]));
+        s[9] = (P[0].d[0] + P[1].d[1]) + tr;
         double th = 0, gf = 0;
         if (active) theta_site<GF_MAG>(s, th, gf);
         th = wave64_sum(th);
@@ -1350,11 +1326,11 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_mag64(GaugeSweepArgs a)
         Philox rng;  // overrelaxation draws no random numbers
         A q[4];
         const auto update = [&](A D, Cx<A> x) { finish_update<A, GF_MAG, GF_OR, false>(D, x.y, x.x, (A)0, q, a.param, rng); };
-        update((A)2 * (P[0].d[0] - P[0].d[2]) + (P[1].d[0] - P[1].d[2]), x02());
+        update(P[0].d[0] - P[0].d[2], x02());
         turn_su2<A, 0, 2>(P[0], q);
         turn_su2<A, 0, 2>(P[1], q);
         left_su2<A, 0, 2>(Gx, q);
-        update((A)2 * (P[1].d[1] - P[1].d[2]) + (P[0].d[1] - P[0].d[2]), x12());
+        update(P[1].d[1] - P[1].d[2], x12());
         turn_su2<A, 1, 2>(P[0], q);
         turn_su2<A, 1, 2>(P[1], q);
         left_su2<A, 1, 2>(Gx, q);
