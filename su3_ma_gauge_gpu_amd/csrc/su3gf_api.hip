@@ -709,14 +709,17 @@ std::array<int, 8> slab_key(const Geom &geo, int gauge, int links, bool fp64)
 }
 
 // the block orders (order_span) that the tuner tries beside the default: the
-// other passes of an XCD's own timeslices, or, where Nt / 8 is not whole, the
-// other divisors of Nt up to 18
-std::vector<int> order_candidates(int Nt)
+// other passes of an XCD's own timeslices, where it has whole ones of whole
+// blocks.  Elsewhere the default is kept untimed: of the divisors of Nt, timed
+// on ten lattices from 6^4 to 36^4, none won by the 3% asked of it, and timing
+// them made a first run of 12^4 38 ms instead of 19, of 36^4 260 instead of 93.
+std::vector<int> order_candidates(const Geom &geo, int block_sites)
 {
     std::vector<int> out;
-    const int def = order_span(Nt, 0), top = Nt % 8 == 0 ? Nt / 8 : std::min(Nt, 18);
-    for (int P = 1; P <= top; P++)
-        if (P != def && order_span(Nt, P) == P) out.push_back(P);
+    const int Nt = geo.N[0], own = Nt / 8;
+    if (Nt % 8 != 0 || geo.Vh / Nt % block_sites != 0) return out;
+    for (int P = 1; P < own; P++)
+        if (own % P == 0) out.push_back(P);
     return out;
 }
 
@@ -794,7 +797,7 @@ GsweepTuning tune_gsweep(const GaugeSweepArgs &ga, int gauge, bool fp64, hipStre
         if (log) std::fprintf(stderr, "su3gf tune:   two kernels, one pass: %.4f ms per sweep (%d sweeps)\n", base, n);
         float two = base;
         if (g_tpass_setting < 0 && base > 0) {
-            for (int P : order_candidates(geo.N[0])) {
+            for (int P : order_candidates(geo, 64)) {
                 t.tpass = P;
                 const float ms = time_gsweep(t, gauge, fp64, 0, n, s, ev.a, ev.b);
                 if (log) std::fprintf(stderr, "su3gf tune:   two kernels, %d timeslices together: %.4f\n", P, ms);
@@ -904,7 +907,9 @@ int quality_tpass(const gf_lattice *lat, int gauge, const void *U, hipStream_t s
                                  gauge};
     const auto hit = g_quality_cache.find(key);
     if (hit != g_quality_cache.end()) return hit->second;
-    const std::vector<int> spans = order_candidates(lat->dims[0]);
+    int64_t V = 1;
+    for (int d = 0; d < 4; d++) V *= lat->dims[d];
+    const std::vector<int> spans = order_candidates(make_geom(lat->dims, V), exact::kQualitySites);
     int best = 0;
     EventPair ev;
     if (!spans.empty() && hipEventCreate(&ev.a) == hipSuccess && hipEventCreate(&ev.b) == hipSuccess) {

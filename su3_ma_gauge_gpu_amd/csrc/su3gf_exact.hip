@@ -426,7 +426,6 @@ __device__ __forceinline__ void quality_site(const QualityArgs<R> &a, int64_t si
     dGff = result;
 }
 
-constexpr int kQualitySites = 128;  // sites of each parity per block
 
 // (theta, gff) of the lattice from its n blocks' partials in a fixed order: sum
 // k (k = 0..1023) takes partials k, k + 1024, ... in order, then a fixed tree.

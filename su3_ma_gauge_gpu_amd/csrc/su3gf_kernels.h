@@ -220,6 +220,7 @@ template <typename R>
 hipError_t launch_project(int stride, R *U, int64_t V, hipStream_t s, const DevState *st = nullptr);
 template <typename R> hipError_t launch_set_hot(R *U, int64_t V, uint32_t seed, uint32_t counter, hipStream_t s);
 template <typename R> hipError_t launch_quality(int stride, int gauge, const QualityArgs<R> &a, hipStream_t s);
+constexpr int kQualitySites = 128;  // sites of each parity per block of the quality kernel
 int64_t quality_blocks(int64_t V);
 }  // namespace exact
 

@@ -1,5 +1,5 @@
 """The host side of a gauge-quality handle, on the CPU, with a stand-in for the
-HIP runtime (tests/stats_host_check.cpp): what a check's kernel needs is in
+HIP runtime (tests/hip_stand_in.h): what a check's kernel needs is in
 place on the check's own stream."""
 import shutil
 import subprocess
