@@ -152,12 +152,18 @@ __global__ __launch_bounds__(kBlock) void k_sweep_rng(SweepArgs<R> a)
     }
 }
 
-// Up to two blocks per CU the registers are there in any case (PARK = false
-// leaves 2 waves per SIMD in FP64) and the copies only lengthen the update.
-// FP64 heatbath half-sweep with the links kept in registers and put aside, and
+// With the links in registers a heatbath in FP64 holds 2 waves per SIMD, so up
+// to two blocks per CU run at once in any case, and the copies only lengthen
+// the update.  FP64 half-sweep with the links in registers and put aside, and
 // with every wave making the update as in k_sweep: Coulomb timeslice 32^3 (256
-// blocks) 15.6, 16.7 and 16.0 us, Landau 16^4 (512) 20.1, 21.3 and 23.3, 20^4
-// (1250) 44.6, 36.6 and 48.6.
+// blocks) 15.6, 16.7 and 16.0 us; Landau 512 blocks 20.5, 22.0 and 24.0, 576
+// 29.1, 24.2 and 32.3, 810 34.1, 27.7 and 40.4, 1250 45.1, 36.4 and 48.6.  In
+// FP32 there are registers for 3 waves (MAG: 4), and the line could lie at 768
+// blocks (1024): 512 blocks 13.6, 14.2 and 14.7 us, 576 16.7, 17.3 and 19.7, 810
+// 22.2, 17.9 and 22.1; MAG 810 21.7 and 22.7, 1125 28.3 and 24.9.  It lies at 512
+// for every type: above it FP32 gives up 4% at most, and a type of its own
+// would need a line for each gauge.  Stochastic relaxation, whose update is
+// short, gives up 7% (FP64 MAG 576 blocks 15.6 and 16.8 us).
 constexpr unsigned kUnparkedBlocks = 512;
 
 template <typename R, int G, int A, int S, bool STREAM> static hipError_t launch_s(const SweepArgs<R> &a, hipStream_t s)
