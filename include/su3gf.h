@@ -343,8 +343,9 @@ gf_status gf_set_pipelined_lag(int lag, int *previous);
  * a pass boundary.  Where Nt is no multiple of 8, groups of n timeslices are
  * walked instead, n a divisor of Nt (up to 8 by default), and each XCD takes
  * an eighth of that sequence.  The results do not depend on the order (the
- * sites of a parity are independent); the time does.  Chosen per lattice
- * shape, gauge and mode by timing, together with the wavefront slab.
+ * sites of a parity are independent); the time does.  Where each XCD has whole
+ * timeslices of whole blocks it is chosen per lattice shape, gauge and mode by
+ * timing, together with the wavefront slab; elsewhere the default is kept.
  * The drop-in quality kernel (gf_stats_quality, gf_quality_per_site) walks
  * the XCDs' timeslices the same way, and its order is tuned on its first
  * launch for a kind of lattice (timing launches read the links and write
@@ -401,6 +402,11 @@ gf_status gf_block_order_choice(const gf_lattice *lat, int gauge, int mode, int 
  *   mode GF_MIXED_FP64: no FP32 phase (switch_precision, refresh and check32
  *     unused): the FP64 phase alone, on the caller's links -- an all-FP64
  *     run, on the gauge-transformation sweep where the volume allows.
+ * The links are taken as they are: rows 0 and 1, the third rebuilt from them.
+ * Those of U should be unitary to double precision (gf_project): from links
+ * unitary to single precision only, the FP64 phase's theta and gff are those
+ * of g U0 g^dagger before the final projection, which moves them by the links'
+ * own rounding (MAG: a run that met 1e-12 returns links of theta 5e-8).
  * The gauge-transformation modes take at most 44,739,200 sites (80^4 fits;
  * GF_ERR_BAD_SHAPE beyond), GF_MIXED_LINKS any volume below 2^31.
  * No reference counterpart (the reference's DPUPDATES is a compile-time

@@ -688,8 +688,8 @@ gf_status gf_run_or(const gf_lattice *lat, void *U, int gauge, float omega, floa
 namespace {
 std::mutex g_slab_mu;
 // per (shape, gauge, link form, arithmetic): the wavefront slab of sweeps
-// without a check (0: two kernels) and the XCD block order (tpass: passes of
-// that many timeslices, 0: one pass)
+// without a check (0: two kernels) and the XCD block order (tpass: its span in
+// timeslices, order_span, 0: the default)
 struct GsweepTuning {
     int slab = 0;
     int tpass = 0;
@@ -697,7 +697,7 @@ struct GsweepTuning {
 };
 std::map<std::array<int, 8>, GsweepTuning> g_slab_cache;
 int g_slab_setting = -1;   // -1 tuned, 0 never, n > 0 fixed (gf_set_wavefront)
-int g_tpass_setting = -1;  // -1 tuned, 0 one pass, n > 0 passes of n timeslices (gf_set_block_order)
+int g_tpass_setting = -1;  // -1 tuned, 0 the default, n > 0 a span of n timeslices (gf_set_block_order)
 int g_lag_setting = -1;    // -1 tuned, n >= 0 the pipelined sweep's extra lag (gf_set_pipelined_lag)
 // extra lags the tuner tries for the pipelined sweep
 constexpr int kPipeLags[] = {192, 256, 384, 512};
@@ -760,8 +760,7 @@ bool tune_log()
 }
 
 // times OR sweeps of each candidate on a scratch copy of g: first the
-// block order of the two-kernel sweep (passes of each divisor of the XCD's
-// timeslices), then, with that order, the wavefront slabs, then the
+// block order of the two-kernel sweep (order_candidates), then, with that order, the wavefront slabs, then the
 // pipelined sweep's lags; a candidate must beat the incumbent by 3% (launch
 // count, noise), and a choice other than the default must beat it again in
 // alternate timings.  Never fails (the defaults on any error).

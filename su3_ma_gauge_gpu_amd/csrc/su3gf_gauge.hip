@@ -1143,7 +1143,9 @@ __global__ __launch_bounds__(kGBlock) void k_gsweep_mag(GaugeSweepArgs a)
 // (P <- G P G^dagger) and on g(x).  The waves thus stop after their products
 // and do not turn their links by the three updates, with one barrier instead of
 // six: checked launch, with every link turned and as here, 12^4 8.8 and 7.6 us,
-// 24^4 42.5 and 33.1, 32^4 138 and 107, 40^4 342 and 271, 48^4 700 and 624.
+// 24^4 42.5 and 33.1, 32^4 138 and 107, 40^4 342 and 271, 48^4 700 and 621;
+// sweep without a check 16^4 21.2 both, 24^4 70.5 and 67.5, 32^4 259 and 207,
+// 40^4 617 and 544, 48^4 1262 and 1243.
 // Sums of links not yet turned by g(x), which wave 0 turns instead (columns 0
 // and 1 only, P_2 = 8 - P_0 - P_1 by unitarity), take 31, 95, 246 and 560 us at
 // 24^4 to 48^4, but they are of order 8 where the turned ones' off-diagonal

@@ -112,7 +112,7 @@ struct GaugeSweepArgs {
     int64_t keep;      // set by the launcher: the links of each parity kept in the Infinity Cache
                        // (kept_link); the two-kernel sweep streams the others
     bool stream_g;     // set by the launcher: the updated sites' own g is streamed too
-    uint32_t seed, counter;  // SA / random transformation (Philox key and counter)
+    uint32_t seed, counter;  // SA (Philox key and counter)
     int64_t nsb;       // sites per block of the reference launch (RNG key)
     int links24;       // U0 in the 24-bit fixed-point form of launch_pack24 (OR, SA, microcanonical)
     int links64;       // U0 and g in FP64 tiles (kTiled12, 12 doubles per site): the mixed driver's
