@@ -587,9 +587,11 @@ gf_status gf_stats_quality(gf_stats *st, const gf_lattice *lat, const void *U, d
     const int crit_max = st->crit == GF_CRIT_MAX;
     // a check that leaves no result reports NaN, not the one before it
     st->host->theta = st->host->gff = std::numeric_limits<double>::quiet_NaN();
-    // the first check zeroes the count on its own stream (the caller's need not
-    // wait for the null stream, nor for a fill made when the handle was)
-    if (!st->counted) HIP_TRY(hipMemsetAsync(st->finished, 0, sizeof(uint32_t), S(stream)));
+    // the first check that counts blocks zeroes the count on its own stream (the
+    // caller's need not wait for the null stream, nor for a fill made when the
+    // handle was)
+    if (!st->counted && st->nblocks <= exact::kSmallQualityBlocks)
+        HIP_TRY(hipMemsetAsync(st->finished, 0, sizeof(uint32_t), S(stream)));
     GF_TRY(quality_launch(lat, st->gauge, U, nullptr, nullptr, st->partial, st, crit_max, S(stream)));
     HIP_TRY(hipStreamSynchronize(S(stream)));
     st->counted = true;

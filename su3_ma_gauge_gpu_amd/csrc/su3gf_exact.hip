@@ -565,7 +565,7 @@ static hipError_t launch_quality_s(int gauge, QualityArgs<R> a, hipStream_t s)
     static_assert(2 * kQualitySites == kBlock, "a block holds both parities' sites");
     a.order = make_block_order(quality_blocks(a.g.V), a.g.N[0], a.tpass);
     const unsigned grid = (unsigned)order_grid(a.order);
-    const bool small = a.order.n <= 256;
+    const bool small = a.order.n <= kSmallQualityBlocks;
     const auto launch = [&](auto G_, auto SMALL_) {
         constexpr int G = decltype(G_)::value;
         hipLaunchKernelGGL((k_quality<R, G, S, decltype(SMALL_)::value>), dim3(grid), dim3(kBlock), 0, s, a);

@@ -222,6 +222,8 @@ template <typename R> hipError_t launch_set_hot(R *U, int64_t V, uint32_t seed, 
 template <typename R> hipError_t launch_quality(int stride, int gauge, const QualityArgs<R> &a, hipStream_t s);
 constexpr int kQualitySites = 128;  // sites of each parity per block of the quality kernel
 int64_t quality_blocks(int64_t V);
+// up to one block per CU the block that ends last reduces the partials (QualityArgs::finished)
+constexpr int64_t kSmallQualityBlocks = 256;
 }  // namespace exact
 
 // fast translation unit (contracted, fused theta, gauge accumulation)
